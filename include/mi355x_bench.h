@@ -187,6 +187,9 @@ int mb_tensor_peak(int format, const mb_peak_config* config, const void* a, uint
 
 /* ---- tensor: dense GEMM ---------------------------------------------------- */
 
+/* The largest tile a launch may use. It uses that tile or, where the shape
+ * runs faster so (few tiles, or a ragged last round of them), a smaller one of
+ * the same format: mb_gemm_launched_kernel names the kernel. */
 typedef struct mb_gemm_config {
   uint32_t tile_m;  /* output rows per workgroup */
   uint32_t tile_n;  /* output columns per workgroup */
@@ -208,10 +211,9 @@ const char* mb_gemm_kernel_name(int format, const mb_gemm_config* config);
  * [b][r][g] scales row r over K elements 256b+32g .. 256b+32g+31 (entries
  * past K are ignored): one 256-element K step of a tile reads one contiguous
  * run of 8 bytes per row. K * element bits must be a multiple of 128 (16-byte
- * rows); other shapes are bounded by a checked kernel variant. group_m = 0
- * selects the variant's default band height (tile rows per band: 8, or the
- * measured best of its fast-path kernel: 4 for BF16 and FP16, 6 for FP8 and 7
- * for INT8 256x256);
+ * rows). group_m = 0 selects the launched kernel's default band height (tile
+ * rows per band: 8, or the measured best of its exact-shape kernel: 4 for BF16
+ * and FP16, 6 for FP8 and 7 for INT8 256x256);
  * a band taller than the tile rows acts as the full height. The band height
  * orders the tiles only: every value gives the same C.
  * Replaces: bench_tensor.py:172-209 (_gemm_kernel) and 235-246 (_launch),
@@ -223,9 +225,9 @@ int mb_gemm(int format, const mb_gemm_config* config, const void* a, uint64_t a_
             uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n, uint32_t k,
             uint32_t group_m, void* stream);
 
-/* Registered name of the kernel mb_gemm launches for this call (the tile's
- * fast kernel, or its "_checked" variant for shapes the fast kernel does not
- * take), for the instruction and resource audit of what actually runs; NULL
+/* Registered name of the kernel mb_gemm launches for this call (of the
+ * requested tile or a smaller one; "_checked" for rows too long for the fast
+ * kernels' 32-bit offsets), for the instruction and resource audit of what actually runs; NULL
  * with mb_last_error() set for an invalid call.
  * Replaces: the CompiledKernel the reference's launch returns for its audit
  * (bench_tensor.py:594-600, 988). */

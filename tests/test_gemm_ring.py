@@ -1,0 +1,159 @@
+"""The ring GEMM kernels at the edges of their tiles, K steps and dispatch, against oracle.tensor.
+
+Operands are exact lattices (FP64: N(0,1) within its tolerance), so the
+comparison is exact. The shapes reach every ring kernel of every format with M
+and N off its tile and K off its 128-byte step (a CPU test pins that).
+"""
+
+import numpy as np
+import pytest
+
+from oracle import tensor as ot
+from test_gpu_gemm import FORMATS, _assert_matches, _configs, _run_gemm, _scale_blocks
+
+CHUNK = {"bf16": 8, "fp16": 8, "fp32": 4, "fp64": 2, "int8": 16, "fp8": 16, "fp4": 32}  # elements per 16 bytes
+# (M, N, 16-byte chunks of K): one element, one step exactly, tails in M, N and K, odd and even step counts;
+# then one shape per larger ring tile.
+SHAPES = [(1, 1, 1), (64, 64, 8), (65, 63, 9), (130, 70, 23), (192, 128, 16), (2040, 2035, 33), (2047, 2049, 9),
+          (2600, 2500, 161)]
+
+
+class _Scales:
+    """Stands in for an aligned device tensor where only the pointer matters."""
+
+    def data_ptr(self):
+        return 4096
+
+    def numel(self):
+        return 1
+
+    def element_size(self):
+        return 1
+
+
+def _launched(dtype, config, m, n, k):
+    from triton_chip_benchmarks_amd import _native
+
+    scales = (_Scales(), _Scales()) if dtype == "fp4" else (None, None)
+    return _native.gemm_launched_kernel(dtype, config, m, n, k, *scales)
+
+
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_shapes_reach_every_ring_kernel(dtype):
+    from triton_chip_benchmarks_amd import _native
+
+    prefix = _native.gemm_kernel_name(dtype, _configs(dtype)[0]).rsplit("_", 1)[0] + "_"
+    ring = {name for name in _native.kernel_names()
+            if name.startswith(prefix) and not name.endswith("_checked")
+            and "_256x256x" not in name and name != "gemm_f64_256x128x16"}
+    seen = {_launched(dtype, config, m, n, chunks * CHUNK[dtype])
+            for config in _configs(dtype) for m, n, chunks in SHAPES}
+    assert ring <= seen, ring - seen
+
+
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_a_launch_never_exceeds_the_requested_tile(dtype):
+    """Whatever the shape, the launched kernel's tile fits inside the requested one, and rows too long for
+    32-bit offsets go to the checked kernel."""
+    for config in _configs(dtype):
+        for m, n, k in [(1, 1, 256), (300, 5000, 512), (4096, 4096, 4096), (8192, 256, 1024)]:
+            tile = _launched(dtype, config, m, n, k).split("_")[2]
+            tile_m, tile_n, _ = (int(x) for x in tile.split("x"))
+            assert tile_m <= config["tile_m"] and tile_n <= config["tile_n"], (config, m, n, k, tile)
+        assert _launched(dtype, config, 64, 64, (1 << 22) * CHUNK[dtype]).endswith("_checked")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", FORMATS)
+@pytest.mark.parametrize("m,n,chunks", SHAPES)
+def test_ring_kernels_match_oracle(gpu, dtype, m, n, chunks):
+    k = chunks * CHUNK[dtype]
+    rng = np.random.default_rng(m + n + k)
+    for launched in sorted({_launched(dtype, config, m, n, k) for config in _configs(dtype)}):
+        config = next(c for c in _configs(dtype) if _launched(dtype, c, m, n, k) == launched)
+        print(f"gemm {dtype} {m}x{n}x{k} via {launched}", flush=True)
+        got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng)
+        _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_ring_kernels_write_only_c_and_read_nothing_past_their_operands(gpu, dtype):
+    """C with guard rows and NaN (INT8: -3) bytes after A, B and the scales: a load past an edge that reached
+    a product would show in C, a store past one in the guard."""
+    import torch
+
+    from triton_chip_benchmarks_amd import _native
+
+    m, n, k = 67, 45, 11 * CHUNK[dtype]
+    rng = np.random.default_rng(5)
+    config = _configs(dtype)[0]
+    scales = (None, None)
+    if dtype == "fp4":
+        codes = [rng.integers(0, 16, (rows, k), dtype=np.uint8) for rows in (m, n)]
+        exponents = [rng.integers(126, 129, (rows, k // 32), dtype=np.uint8) for rows in (m, n)]
+        values = [ot.e2m1_decode(c) * np.repeat(ot.e8m0_decode(s), 32, axis=1) for c, s in zip(codes, exponents)]
+        blocks = [_scale_blocks(s) for s in exponents]
+        for block in blocks:
+            block[-1][:, (k // 32) % 8:] = 255  # the caller's padding: E8M0 NaN
+        scales = tuple(torch.from_numpy(block).cuda() for block in blocks)
+        a, b = (torch.from_numpy(ot.pack_e2m1(c)).cuda() for c in codes)
+    else:
+        _, *values, (_, a, b) = _run_gemm(dtype, config, m, n, k, rng, keep_device=True)
+    poisoned = []
+    for tensor in (a, b):
+        poison = torch.full((tensor.numel() * tensor.element_size() + 4096,), 0xFF, dtype=torch.uint8, device="cuda")
+        poison[:tensor.numel() * tensor.element_size()] = tensor.reshape(-1).view(torch.uint8)
+        poisoned.append(poison)
+    out = torch.int32 if dtype == "int8" else torch.float64 if dtype == "fp64" else torch.float32
+    c = torch.full((m + 70, n), -3, dtype=out, device="cuda")
+    _native.gemm(dtype, config, *poisoned, c, m, n, k, *scales)
+    torch.cuda.synchronize()
+    got = c.cpu().numpy().astype(np.float64)
+    _assert_matches(dtype, got[:m], ot.gemm_reference(values[0], values[1].T))
+    assert (got[m:] == -3).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "fp64", "fp8"])
+def test_rows_past_the_32_bit_offsets_run_the_checked_kernel(gpu, dtype):
+    """64 rows of 2^25 bytes are the first that a 64x64 tile cannot address with 31-bit offsets."""
+    m, n, k = 3, 2, (1 << 21) * CHUNK[dtype]
+    config = _configs(dtype)[0]
+    assert _launched(dtype, config, m, n, k).endswith("_checked")
+    print(f"gemm {dtype} {m}x{n}x{k} via {_launched(dtype, config, m, n, k)}", flush=True)
+    got, a_values, b_values = _run_gemm(dtype, config, m, n, k, np.random.default_rng(3))
+    reference = ot.gemm_reference(a_values, b_values.T)
+    if dtype == "fp64":
+        # Forward bound of K serial FMAs: K * 2^-53 * sum |a b|, here about 1e-9 of the sum.
+        allowed = k * 2.0**-53 * ot.gemm_reference(np.abs(a_values), np.abs(b_values).T)
+        assert np.all(np.abs(got - reference) <= allowed)
+    else:
+        _assert_matches(dtype, got, reference)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("offset,checked", [(1, True), (4, False)])
+def test_mxfp4_scales_off_the_16_byte_grid(gpu, offset, checked):
+    """Scales on a dword take the ring kernel's DMAs, byte-aligned ones the checked kernel."""
+    import torch
+
+    from triton_chip_benchmarks_amd import _native
+
+    m, n, k = 70, 33, 544
+    rng = np.random.default_rng(offset)
+    codes = [rng.integers(0, 16, (rows, k), dtype=np.uint8) for rows in (m, n)]
+    exponents = [rng.integers(126, 129, (rows, k // 32), dtype=np.uint8) for rows in (m, n)]
+    values = [ot.e2m1_decode(c) * np.repeat(ot.e8m0_decode(s), 32, axis=1) for c, s in zip(codes, exponents)]
+    scales = []
+    for block in map(_scale_blocks, exponents):
+        flat = torch.from_numpy(np.concatenate([np.zeros(offset, np.uint8), block.reshape(-1)])).cuda()
+        scales.append(flat[offset:])
+    config = _configs("fp4")[0]
+    name = _native.gemm_launched_kernel("fp4", config, m, n, k, *scales)
+    assert name.endswith("_checked") == checked
+    print(f"gemm fp4 scale offset {offset} via {name}", flush=True)
+    c = torch.full((m, n), float("nan"), device="cuda")
+    _native.gemm("fp4", config, *(torch.from_numpy(ot.pack_e2m1(x)).cuda() for x in codes), c, m, n, k, *scales)
+    torch.cuda.synchronize()
+    assert np.array_equal(c.cpu().numpy().astype(np.float64), ot.gemm_reference(values[0], values[1].T))

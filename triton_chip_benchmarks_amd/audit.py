@@ -28,7 +28,8 @@ MATRIX_MNEMONICS = ("v_mfma_", "v_wmma_", "v_mmac_")
 _MFMA_FORMAT = {"MfmaBf16": "bf16", "MfmaF16": "f16", "MfmaI8": "i8", "MfmaFp8": "fp8",
                 "MfmaMxfp4": "mxfp4", "MfmaF32": "f32", "MfmaF64": "f64"}
 _PEAK_RE = re.compile(r"tensor_peak_(?:tied_)?kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])E")
-_GEMM_RE = re.compile(r"gemm_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])E")
+_GEMM_RE = re.compile(r"gemm_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E")
+_GEMM_RING_RE = re.compile(r"gemm_ring_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)EE")
 _GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)EE")
 _ELEM_BITS = {"bf16": 16, "f16": 16, "i8": 8, "fp8": 8, "mxfp4": 4, "f32": 32, "f64": 64}
 _COPY_RE = re.compile(r"copy_kernelI(Dv4_j|j|h)Li(\d+)ELi([012])E")
@@ -36,6 +37,13 @@ _READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)Li(\d+)E")
 _VECTOR_RE = re.compile(r"vector_(\w+?)_kernelILi(\d+)E")
 _COPY_UNIT = {"Dv4_j": "dwordx4", "j": "dword", "h": "byte"}
 _READ_TYPE = {"f": "f32", "DF16_": "f16", "t": "bf16"}
+
+
+def ring_name(op: str, bm: str, bn: str, stages: str) -> str:
+    """Registry name of a ring GEMM kernel: the 128x128 tile with two stages, of which a CU holds a pair, is marked."""
+    fmt = _MFMA_FORMAT[op]
+    pair = "_pair" if (bm, stages) == ("128", "2") else ""
+    return f"gemm_{fmt}_{bm}x{bn}x{128 * 8 // _ELEM_BITS[fmt]}{pair}"
 
 
 def registered_name(symbol: str) -> str | None:
@@ -48,8 +56,11 @@ def registered_name(symbol: str) -> str | None:
                 f"{'nk' if nk == '1' else 'kn'}")
     match = _GEMM_RE.search(symbol)
     if match:
-        op, bm, bn, bk, _wm, _wn, checked = match.groups()
-        return f"gemm_{_MFMA_FORMAT[op]}_{bm}x{bn}x{bk}{'_checked' if checked == '1' else ''}"
+        op, bm, bn, bk, _wm, _wn = match.groups()
+        return f"gemm_{_MFMA_FORMAT[op]}_{bm}x{bn}x{bk}_checked"
+    match = _GEMM_RING_RE.search(symbol)
+    if match:
+        return ring_name(*match.groups())
     match = _GEMM_STAGED_RE.search(symbol)
     if match:
         fmt = _MFMA_FORMAT[match.group(1).removesuffix("x16")]

@@ -123,8 +123,12 @@ def registered_name(demangled: str) -> str:
         return (f"tensor_peak_{_MFMA_FORMAT[fmt.removesuffix('x16')]}_{bm}x{bn}x{bk}_c{chains}{shape}_"
                 f"{'nk' if nk in ('true', '1') else 'kn'}")
     if family == "gemm_kernel":
-        fmt, bm, bn, bk, _wm, _wn, checked = args
-        return f"gemm_{_MFMA_FORMAT[fmt]}_{bm}x{bn}x{bk}{'_checked' if checked in ('true', '1') else ''}"
+        fmt, bm, bn, bk = args[:4]
+        return f"gemm_{_MFMA_FORMAT[fmt]}_{bm}x{bn}x{bk}_checked"
+    if family == "gemm_ring_kernel":
+        from .audit import ring_name
+
+        return ring_name(*args)
     if family in ("gemm_staged_kernel", "gemm_dma_kernel"):
         name = _MFMA_FORMAT[args[0].removesuffix("x16")]
         return f"gemm_{name}_256x256x{128 * 8 // _ELEM_BITS[name]}"

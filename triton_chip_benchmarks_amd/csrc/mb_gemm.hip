@@ -12,27 +12,33 @@
 // row-major; the MI355X kernel takes K-contiguous B (layout prepared outside
 // timing by the caller).
 //
-// Two kernels:
-//   * gemm_dma_kernel (BF16, FP16, INT8, FP8 on 16x16 MFMAs) and
-//     gemm_staged_kernel (MXFP4): 256x256 tiles when the shape divides the
-//     tile. Four waves, one per SIMD, each owning 128x128 outputs in AGPRs:
-//     64 accumulators of 16x16 (the 16x16 instructions sustain a higher clock
-//     under the power limit) or, for MXFP4, 16 of 32x32. In the staged kernel
-//     operands flow global -> VGPR -> LDS -> VGPR -> MFMA: each K step (128
-//     bytes of every row) is loaded two steps ahead into one of two register
-//     sets, written to one of two LDS stages a step ahead, and read back as
-//     fragments ahead of the MFMAs that use them. Loads, stage writes and
-//     fragment reads are spread across the step's MFMAs, so no burst of
-//     memory instructions stalls the in-order MFMA issue; one barrier per
-//     step. The DMA kernel moves A straight into LDS with LDS-DMA loads
-//     instead.
-//   * gemm_kernel: every other tile and every ragged shape (CHECKED
-//     instantiations bound each load and store), operands staged through a
-//     padded, double-buffered LDS tile with 16-byte loads.
-// Both number workgroups XCD-first: the hardware deals consecutive ids
-// round-robin over the 8 XCDs, so id i is remapped to the i/8-th tile of XCD
-// i%8's contiguous share, walked in GROUP_M-row bands that keep A and B panels
-// hot in that XCD's L2.
+// Three families, of which a launch uses the one estimated fastest (gemm_cost)
+// among those with tiles no larger than the caller asked for:
+//   * gemm_dma_kernel (BF16, FP16, INT8, FP8, FP32 on 16x16 MFMAs),
+//     gemm_dma_f64_kernel and gemm_staged_kernel (MXFP4): 256x256 tiles
+//     (FP64 256x128) when the shape divides the tile. Four waves, one per SIMD,
+//     each owning 128x128 outputs in AGPRs: 64 accumulators of 16x16 (the 16x16
+//     instructions sustain a higher clock under the power limit) or, for MXFP4,
+//     16 of 32x32. In the staged kernel operands flow global -> VGPR -> LDS ->
+//     VGPR -> MFMA: each K step (128 bytes of every row) is loaded two steps
+//     ahead into one of two register sets, written to one of two LDS stages a
+//     step ahead, and read back as fragments ahead of the MFMAs that use them.
+//     Loads, stage writes and fragment reads are spread across the step's
+//     MFMAs, so no burst of memory instructions stalls the in-order MFMA issue;
+//     one barrier per step. The DMA kernels move A straight into LDS with
+//     LDS-DMA loads instead.
+//   * gemm_ring_kernel (mb_gemm_ring.h): 64x64, 128x128 and 256x128 tiles, any
+//     shape. Large tiles leave CUs idle on small problems: 2048^3 in BF16 has
+//     64 tiles of 256x256 (39.3 us) but 256 of 128x128 (20.4 us).
+//   * gemm_kernel: 128x128 tiles staged through registers into a padded,
+//     double-buffered LDS tile, every load and store bounded with 64-bit
+//     addresses: rows too long for the other families' 32-bit offsets.
+// All number workgroups XCD-first: the hardware deals consecutive ids
+// round-robin over the 8 XCDs, so ids are remapped to give each XCD a
+// contiguous share, walked in GROUP_M-row bands that keep A and B panels hot
+// in that XCD's L2.
+#include "mb_gemm_device.h"
+#include "mb_gemm_host.h"
 #include "mb_internal.h"
 #include "mb_mfma.h"
 
@@ -41,8 +47,6 @@
 
 namespace mb {
 namespace {
-
-constexpr int kXcds = 8;
 
 template <class Op, int BM, int BN, int BK, int WAVES_M, int WAVES_N>
 struct GemmTile {
@@ -63,7 +67,7 @@ struct GemmTile {
 };
 
 // Stage one K step of A and B into registers (global loads in flight).
-template <class T, bool CHECKED>
+template <class T>
 __device__ __forceinline__ void load_step(i32x4 (&ra)[T::A_CHUNKS], i32x4 (&rb)[T::B_CHUNKS],
                                           const uint8_t* a_tile, const uint8_t* b_tile, uint64_t row_bytes,
                                           int rows_a, int rows_b, int64_t k_bytes_left) {
@@ -72,7 +76,7 @@ __device__ __forceinline__ void load_step(i32x4 (&ra)[T::A_CHUNKS], i32x4 (&rb)[
   for (int i = 0; i < T::A_CHUNKS; ++i) {
     const int c = i * T::THREADS + t;
     const int row = c / T::ROW_CHUNKS, chunk = c % T::ROW_CHUNKS;
-    if (!CHECKED || (row < rows_a && chunk * 16 < k_bytes_left))
+    if (row < rows_a && chunk * 16 < k_bytes_left)
       ra[i] = *reinterpret_cast<const i32x4*>(a_tile + row * row_bytes + chunk * 16);
     else
       ra[i] = i32x4{0, 0, 0, 0};
@@ -81,7 +85,7 @@ __device__ __forceinline__ void load_step(i32x4 (&ra)[T::A_CHUNKS], i32x4 (&rb)[
   for (int i = 0; i < T::B_CHUNKS; ++i) {
     const int c = i * T::THREADS + t;
     const int row = c / T::ROW_CHUNKS, chunk = c % T::ROW_CHUNKS;
-    if (!CHECKED || (row < rows_b && chunk * 16 < k_bytes_left))
+    if (row < rows_b && chunk * 16 < k_bytes_left)
       rb[i] = *reinterpret_cast<const i32x4*>(b_tile + row * row_bytes + chunk * 16);
     else
       rb[i] = i32x4{0, 0, 0, 0};
@@ -105,7 +109,7 @@ __device__ __forceinline__ void store_step(uint8_t* buffer, const i32x4 (&ra)[T:
   }
 }
 
-template <class Op, int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool CHECKED>
+template <class Op, int BM, int BN, int BK, int WAVES_M, int WAVES_N>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
     gemm_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__ SA,
                 const uint8_t* __restrict__ SB, typename Op::Out* __restrict__ C, int M, int N, int K,
@@ -148,7 +152,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
     for (int tn = 0; tn < T::TN; ++tn) acc[tm][tn] = typename Op::Acc{};
 
   i32x4 ra[T::A_CHUNKS], rb[T::B_CHUNKS];
-  load_step<T, CHECKED>(ra, rb, a_tile, b_tile, row_bytes, rows_a, rows_b, static_cast<int64_t>(row_bytes));
+  load_step<T>(ra, rb, a_tile, b_tile, row_bytes, rows_a, rows_b, static_cast<int64_t>(row_bytes));
   store_step<T>(lds, ra, rb, BM);
   __syncthreads();
 
@@ -156,7 +160,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
     uint8_t* current = lds + (kt & 1) * T::BUFFER;
     const bool more = kt + 1 < k_steps;
     if (more)
-      load_step<T, CHECKED>(ra, rb, a_tile + (kt + 1) * T::BK_BYTES, b_tile + (kt + 1) * T::BK_BYTES, row_bytes,
+      load_step<T>(ra, rb, a_tile + (kt + 1) * T::BK_BYTES, b_tile + (kt + 1) * T::BK_BYTES, row_bytes,
                             rows_a, rows_b, static_cast<int64_t>(row_bytes) - (kt + 1) * T::BK_BYTES);
     // E8M0 scales of this step: column kt*BK/32 + ks*LANE_GROUPS + group.
     int sa[T::TM][T::KSTEPS], sb[T::TN][T::KSTEPS];
@@ -167,7 +171,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
         for (int ks = 0; ks < T::KSTEPS; ++ks) {
           const int row = m0 + wm * T::WM + tm * Op::M + lrow;
           const int col = kt * T::GROUPS + ks * MfmaGeometry<Op>::LANE_GROUPS + lgroup;
-          sa[tm][ks] = (!CHECKED || (row < M && col < scale_cols)) ? scale_at(SA, M, row, col) : 127;
+          sa[tm][ks] = row < M && col < scale_cols ? scale_at(SA, M, row, col) : 127;
         }
 #pragma unroll
       for (int tn = 0; tn < T::TN; ++tn)
@@ -175,7 +179,7 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
         for (int ks = 0; ks < T::KSTEPS; ++ks) {
           const int col_n = n0 + wn * T::WN + tn * Op::N + lrow;
           const int col = kt * T::GROUPS + ks * MfmaGeometry<Op>::LANE_GROUPS + lgroup;
-          sb[tn][ks] = (!CHECKED || (col_n < N && col < scale_cols)) ? scale_at(SB, N, col_n, col) : 127;
+          sb[tn][ks] = col_n < N && col < scale_cols ? scale_at(SB, N, col_n, col) : 127;
         }
     } else {
 #pragma unroll
@@ -214,61 +218,8 @@ __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
       for (int r = 0; r < Op::ACC_REGS; ++r) {
         const int row = m0 + wm * T::WM + tm * Op::M + Op::out_row(lane, r);
         const int col = n0 + wn * T::WN + tn * Op::N + (lane % Op::N);
-        if (!CHECKED || (row < M && col < N)) C[static_cast<int64_t>(row) * N + col] = acc[tm][tn][r];
+        if (row < M && col < N) C[static_cast<int64_t>(row) * N + col] = acc[tm][tn][r];
       }
-}
-
-// ---- shared pieces of the 256x256 kernels ---------------------------------
-
-// One 16-byte-per-lane LDS DMA: lane l's 16 bytes land at lds_addr + 16 * l.
-// Issued as inline assembly so the compiler's wait-count pass does not force a
-// full vmcnt(0) before every LDS read; the staged kernel issues it ahead of
-// compiler-visible loads, whose in-order vmcnt waits then cover it.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset, uint32_t lds_addr) {
-  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(rsrc), "s"(soffset),
-               "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr))
-               : "memory");
-}
-
-// Word 3 of a gfx9 buffer resource: 32-bit data format, no swizzle, raw offsets.
-constexpr int kBufferWord3 = 0x00020000;
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const uint8_t* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, bytes, kBufferWord3);
-}
-
-// Tile (tile_m, tile_n) of workgroup blockIdx.x: XCD-first numbering, then
-// GROUP_M-row bands (see the file comment).
-__device__ __forceinline__ void band_tile(int tiles_m, int tiles_n, int group_m, int& tile_m, int& tile_n) {
-  const int count = gridDim.x;
-  int pid = blockIdx.x;
-  if (count % kXcds == 0) pid = (pid % kXcds) * (count / kXcds) + pid / kXcds;
-  const int band = group_m * tiles_n;
-  const int first_m = (pid / band) * group_m;
-  const int rows_in_band = min(tiles_m - first_m, group_m);
-  tile_m = first_m + (pid % band) % rows_in_band;
-  tile_n = (pid % band) / rows_in_band;
-}
-
-// s_waitcnt's immediate for vmcnt(n) alone (n < 64): vmcnt's low four bits
-// at 3:0 and high two at 15:14, expcnt (6:4) and lgkmcnt (11:8) at their
-// maxima, which wait for nothing.
-constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
-
-// Barrier that orders LDS only: global loads in flight stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// f(integral_constant<I>) for I = I0 .. N-1, so counts derived from I are constants.
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
 }
 
 // ---- VGPR-staged 256x256 kernel (MXFP4) ------------------------------------
@@ -870,26 +821,19 @@ __global__ void __launch_bounds__(256)
 #endif
 }
 
-// Launchers size their own grid: one workgroup per output tile of their kernel.
-using GemmLauncher = void (*)(const uint8_t*, const uint8_t*, const uint8_t*, const uint8_t*, void*, int, int, int,
-                              int, hipStream_t);
-
-inline uint32_t tile_count(int m, int n, int bm, int bn) {
-  return static_cast<uint32_t>(((m + bm - 1) / bm) * static_cast<int64_t>((n + bn - 1) / bn));
-}
-
-template <class Op, int BM, int BN, int BK, int WM, int WN, bool CHECKED>
-void launch_gemm(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m, int n,
-                 int k, int group_m, hipStream_t stream) {
-  gemm_kernel<Op, BM, BN, BK, WM, WN, CHECKED><<<dim3(tile_count(m, n, BM, BN)), dim3(64 * WM * WN), 0, stream>>>(
+template <class Op>
+void launch_checked(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m, int n,
+                    int k, int group_m, hipStream_t stream) {
+  constexpr int BK = 128 * 8 / Op::ELEM_BITS;
+  gemm_kernel<Op, 128, 128, BK, 2, 2><<<dim3(tile_count(m, n, 128, 128)), dim3(256), 0, stream>>>(
       a, b, sa, sb, static_cast<typename Op::Out*>(c), m, n, k, group_m);
 }
 
-// The fast-path kernel of an instruction: the all-DMA kernel for the unscaled
+// The exact-shape kernel of an instruction: the all-DMA kernel for the unscaled
 // ones (256x256; its 256x128 FP64 form), the register-staged kernel (with its
 // scale ring) for MXFP4.
 template <class Op>
-constexpr auto fast_kernel_fn() {
+constexpr auto exact_kernel_fn() {
   if constexpr (Op::SCALED)
     return gemm_staged_kernel<Op>;
   else if constexpr (Op::ELEM_BITS == 64)
@@ -898,116 +842,93 @@ constexpr auto fast_kernel_fn() {
     return gemm_dma_kernel<Op>;
 }
 
-// Tile width of the fast-path kernel (its height is 256).
+// Tile width of the exact-shape kernel (its height is 256).
 template <class Op>
-constexpr int fast_tile_n() {
+constexpr int exact_tile_n() {
   return Op::ELEM_BITS == 64 ? 128 : 256;
 }
 
 template <class Op>
-const void* fast_kernel() {
-  return reinterpret_cast<const void*>(fast_kernel_fn<Op>());
-}
-
-template <class Op>
-void launch_gemm_staged(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m,
-                        int n, int k, int group_m, hipStream_t stream) {
-  fast_kernel_fn<Op>()<<<dim3(tile_count(m, n, 256, fast_tile_n<Op>())), dim3(256), 0, stream>>>(
+void launch_exact(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m, int n,
+                  int k, int group_m, hipStream_t stream) {
+  exact_kernel_fn<Op>()<<<dim3(tile_count(m, n, 256, exact_tile_n<Op>())), dim3(256), 0, stream>>>(
       a, b, sa, sb, static_cast<typename Op::Out*>(c), m, n, k, group_m);
 }
 
-// What a variant's fast launcher needs beyond a shape that divides its tile.
-enum GemmPath { kLdsPath = 0, kStagedPath = 1 };
+// Exact-shape kernels: GROUP is the band height the sweeps at the benchmark
+// sizes measured best (BF16 and FP16 4, FP8 6, INT8 7, MXFP4 8; FP64 flat, 8).
+#define MB_EXACT(FMT, OP, GROUP, COST, NAME)                                                              \
+  GemmKernel {                                                                                            \
+    FMT, 256, exact_tile_n<OP>(), GROUP, 1, COST, NAME, reinterpret_cast<const void*>(exact_kernel_fn<OP>()), \
+        launch_exact<OP>                                                                                  \
+  }
+const GemmKernel kExactKernels[] = {
+    MB_EXACT(MB_MATRIX_BF16, MfmaBf16x16, 4, kCost256, "gemm_bf16_256x256x64"),
+    MB_EXACT(MB_MATRIX_F16, MfmaF16x16, 4, kCost256, "gemm_f16_256x256x64"),
+    MB_EXACT(MB_MATRIX_FP8_E4M3, MfmaFp8x16, 6, kCost256, "gemm_fp8_256x256x128"),
+    MB_EXACT(MB_MATRIX_I8, MfmaI8x16, 7, kCost256, "gemm_i8_256x256x128"),
+    MB_EXACT(MB_MATRIX_MXFP4, MfmaMxfp4, 8, kCost256, "gemm_mxfp4_256x256x256"),
+    MB_EXACT(MB_MATRIX_F64, MfmaF64, 8, kCostF64x256, "gemm_f64_256x128x16"),
+    MB_EXACT(MB_MATRIX_F32, MfmaF32x16, 8, kCostF32x256, "gemm_f32_256x256x32"),
+};
 
-// launch: shapes that divide the tile and satisfy the path's rule (see
-// exact_shape); launch_checked: any shape.
+// Any shape whose rows are too long for the ring kernels' 32-bit offsets.
+#define MB_CHECKED(FMT, OP, NAME)                                                                             \
+  GemmKernel {                                                                                                \
+    FMT, 128, 128, 8, 1, GemmCost{}, NAME,                                                                    \
+        reinterpret_cast<const void*>(gemm_kernel<OP, 128, 128, 128 * 8 / OP::ELEM_BITS, 2, 2>), launch_checked<OP> \
+  }
+const GemmKernel kCheckedKernels[] = {
+    MB_CHECKED(MB_MATRIX_BF16, MfmaBf16, "gemm_bf16_128x128x64_checked"),
+    MB_CHECKED(MB_MATRIX_F16, MfmaF16, "gemm_f16_128x128x64_checked"),
+    MB_CHECKED(MB_MATRIX_FP8_E4M3, MfmaFp8, "gemm_fp8_128x128x128_checked"),
+    MB_CHECKED(MB_MATRIX_I8, MfmaI8, "gemm_i8_128x128x128_checked"),
+    MB_CHECKED(MB_MATRIX_MXFP4, MfmaMxfp4, "gemm_mxfp4_128x128x256_checked"),
+    MB_CHECKED(MB_MATRIX_F64, MfmaF64, "gemm_f64_128x128x16_checked"),
+    MB_CHECKED(MB_MATRIX_F32, MfmaF32, "gemm_f32_128x128x32_checked"),
+};
+
+// The tiles a caller can ask for. `name` is the kernel of that tile; a launch
+// uses it or, where the shape runs faster so, a kernel with a smaller tile.
 struct GemmVariant {
   int format;
   mb_gemm_config config;
   const char* name;
-  const void* kernel;
-  GemmLauncher launch;
-  GemmLauncher launch_checked;
   int out_bytes;
   int elem_bits;
-  int path;
-  const char* checked_name;
-  const void* checked_kernel;
-  int default_group;  // band height in tile rows when the caller passes 0 (measured per kernel)
 };
-
-#define MB_GEMM(FMT, OP, BM, BN, BK, WM, WN, NAME)                                                           \
-  GemmVariant{FMT,                                                                                           \
-              mb_gemm_config{BM, BN, BK, 64 * WM * WN},                                                      \
-              NAME,                                                                                          \
-              reinterpret_cast<const void*>(gemm_kernel<OP, BM, BN, BK, WM, WN, false>),                     \
-              launch_gemm<OP, BM, BN, BK, WM, WN, false>,                                                    \
-              launch_gemm<OP, BM, BN, BK, WM, WN, true>,                                                     \
-              static_cast<int>(sizeof(typename OP::Out)),                                                    \
-              OP::ELEM_BITS,                                                                                 \
-              kLdsPath,                                                                                      \
-              NAME "_checked",                                                                               \
-              reinterpret_cast<const void*>(gemm_kernel<OP, BM, BN, BK, WM, WN, true>),                      \
-              8}
-
-// 256x256 tiles (256x128 for FP64): the fast-path kernel (BK = 128 bytes of K;
-// instruction SOP) for exact shapes, a checked LDS-staged kernel (tile CM x CN,
-// instruction OP) for the rest.
-#define MB_GEMM_STAGED(FMT, SOP, OP, BK, CM, CN, GROUP, NAME, CNAME)                                              \
-  GemmVariant{FMT,                                                                                           \
-              mb_gemm_config{256, fast_tile_n<SOP>(), BK, 256},                                              \
-              NAME,                                                                                          \
-              fast_kernel<SOP>(),                                                                            \
-              launch_gemm_staged<SOP>,                                                                       \
-              launch_gemm<OP, CM, CN, BK, 2, 2, true>,                                                       \
-              static_cast<int>(sizeof(typename OP::Out)),                                                    \
-              OP::ELEM_BITS,                                                                                 \
-              kStagedPath,                                                                                   \
-              CNAME,                                                                                         \
-              reinterpret_cast<const void*>(gemm_kernel<OP, CM, CN, BK, 2, 2, true>),                        \
-              GROUP}
-// GROUP: the band height the sweeps at the benchmark sizes measured best per
-// fast-path kernel (BF16 and FP16 4, FP8 6, INT8 7, MXFP4 8; FP64 flat, 8).
+#define MB_TILE(FMT, OP, TM, TN, NAME)                                                                       \
+  GemmVariant {                                                                                              \
+    FMT, mb_gemm_config{TM, TN, 128 * 8 / OP::ELEM_BITS, 256}, NAME, static_cast<int>(sizeof(typename OP::Out)), \
+        OP::ELEM_BITS                                                                                        \
+  }
 const GemmVariant kGemmVariants[] = {
-    MB_GEMM_STAGED(MB_MATRIX_BF16, MfmaBf16x16, MfmaBf16, 64, 256, 256, 4, "gemm_bf16_256x256x64",
-                   "gemm_bf16_256x256x64_checked"),
-    MB_GEMM(MB_MATRIX_BF16, MfmaBf16, 256, 128, 64, 2, 2, "gemm_bf16_256x128x64"),
-    MB_GEMM(MB_MATRIX_BF16, MfmaBf16, 128, 128, 64, 2, 2, "gemm_bf16_128x128x64"),
-    MB_GEMM_STAGED(MB_MATRIX_F16, MfmaF16x16, MfmaF16, 64, 256, 256, 4, "gemm_f16_256x256x64",
-                   "gemm_f16_256x256x64_checked"),
-    MB_GEMM(MB_MATRIX_F16, MfmaF16, 256, 128, 64, 2, 2, "gemm_f16_256x128x64"),
-    MB_GEMM(MB_MATRIX_F16, MfmaF16, 128, 128, 64, 2, 2, "gemm_f16_128x128x64"),
-    MB_GEMM_STAGED(MB_MATRIX_FP8_E4M3, MfmaFp8x16, MfmaFp8, 128, 256, 256, 6, "gemm_fp8_256x256x128",
-                   "gemm_fp8_256x256x128_checked"),
-    MB_GEMM(MB_MATRIX_FP8_E4M3, MfmaFp8, 256, 128, 128, 2, 2, "gemm_fp8_256x128x128"),
-    MB_GEMM(MB_MATRIX_FP8_E4M3, MfmaFp8, 128, 128, 128, 2, 2, "gemm_fp8_128x128x128"),
-    MB_GEMM_STAGED(MB_MATRIX_I8, MfmaI8x16, MfmaI8, 128, 256, 256, 7, "gemm_i8_256x256x128",
-                   "gemm_i8_256x256x128_checked"),
-    MB_GEMM(MB_MATRIX_I8, MfmaI8, 256, 128, 128, 2, 2, "gemm_i8_256x128x128"),
-    MB_GEMM(MB_MATRIX_I8, MfmaI8, 128, 128, 128, 2, 2, "gemm_i8_128x128x128"),
-    MB_GEMM_STAGED(MB_MATRIX_MXFP4, MfmaMxfp4, MfmaMxfp4, 256, 128, 128, 8, "gemm_mxfp4_256x256x256",
-                   "gemm_mxfp4_128x128x256_checked"),
-    MB_GEMM(MB_MATRIX_MXFP4, MfmaMxfp4, 256, 128, 256, 2, 2, "gemm_mxfp4_256x128x256"),
-    MB_GEMM(MB_MATRIX_MXFP4, MfmaMxfp4, 128, 128, 256, 2, 2, "gemm_mxfp4_128x128x256"),
-    MB_GEMM_STAGED(MB_MATRIX_F64, MfmaF64, MfmaF64, 16, 128, 128, 8, "gemm_f64_256x128x16",
-                   "gemm_f64_128x128x16_checked"),
-    MB_GEMM(MB_MATRIX_F64, MfmaF64, 128, 128, 16, 2, 2, "gemm_f64_128x128x16"),
-    MB_GEMM(MB_MATRIX_F64, MfmaF64, 64, 64, 16, 2, 2, "gemm_f64_64x64x16"),
-    MB_GEMM_STAGED(MB_MATRIX_F32, MfmaF32x16, MfmaF32, 32, 128, 128, 8, "gemm_f32_256x256x32",
-                   "gemm_f32_128x128x32_checked"),
-    MB_GEMM(MB_MATRIX_F32, MfmaF32, 128, 128, 32, 2, 2, "gemm_f32_128x128x32"),
+    MB_TILE(MB_MATRIX_BF16, MfmaBf16, 256, 256, "gemm_bf16_256x256x64"),
+    MB_TILE(MB_MATRIX_BF16, MfmaBf16, 256, 128, "gemm_bf16_256x128x64"),
+    MB_TILE(MB_MATRIX_BF16, MfmaBf16, 128, 128, "gemm_bf16_128x128x64"),
+    MB_TILE(MB_MATRIX_F16, MfmaF16, 256, 256, "gemm_f16_256x256x64"),
+    MB_TILE(MB_MATRIX_F16, MfmaF16, 256, 128, "gemm_f16_256x128x64"),
+    MB_TILE(MB_MATRIX_F16, MfmaF16, 128, 128, "gemm_f16_128x128x64"),
+    MB_TILE(MB_MATRIX_FP8_E4M3, MfmaFp8, 256, 256, "gemm_fp8_256x256x128"),
+    MB_TILE(MB_MATRIX_FP8_E4M3, MfmaFp8, 256, 128, "gemm_fp8_256x128x128"),
+    MB_TILE(MB_MATRIX_FP8_E4M3, MfmaFp8, 128, 128, "gemm_fp8_128x128x128"),
+    MB_TILE(MB_MATRIX_I8, MfmaI8, 256, 256, "gemm_i8_256x256x128"),
+    MB_TILE(MB_MATRIX_I8, MfmaI8, 256, 128, "gemm_i8_256x128x128"),
+    MB_TILE(MB_MATRIX_I8, MfmaI8, 128, 128, "gemm_i8_128x128x128"),
+    MB_TILE(MB_MATRIX_MXFP4, MfmaMxfp4, 256, 256, "gemm_mxfp4_256x256x256"),
+    MB_TILE(MB_MATRIX_MXFP4, MfmaMxfp4, 256, 128, "gemm_mxfp4_256x128x256"),
+    MB_TILE(MB_MATRIX_MXFP4, MfmaMxfp4, 128, 128, "gemm_mxfp4_128x128x256"),
+    MB_TILE(MB_MATRIX_F64, MfmaF64, 256, 128, "gemm_f64_256x128x16"),
+    MB_TILE(MB_MATRIX_F64, MfmaF64, 128, 128, "gemm_f64_128x128x16"),
+    MB_TILE(MB_MATRIX_F64, MfmaF64, 64, 64, "gemm_f64_64x64x16"),
+    MB_TILE(MB_MATRIX_F32, MfmaF32, 256, 256, "gemm_f32_256x256x32"),
+    MB_TILE(MB_MATRIX_F32, MfmaF32, 128, 128, "gemm_f32_128x128x32"),
 };
 
 struct GemmRegistrar {
   GemmRegistrar() {
-    for (const auto& variant : kGemmVariants) {
-      register_kernel(variant.name, variant.kernel);
-      // A fallback can be another variant's checked kernel: register each name once.
-      bool seen = false;
-      for (const auto* other = kGemmVariants; other != &variant; ++other)
-        seen = seen || std::strcmp(other->checked_name, variant.checked_name) == 0;
-      if (!seen) register_kernel(variant.checked_name, variant.checked_kernel);
-    }
+    for (const GemmKernel& kernel : kExactKernels) register_kernel(kernel.name, kernel.kernel);
+    for (const GemmKernel& kernel : kCheckedKernels) register_kernel(kernel.name, kernel.kernel);
   }
 };
 const GemmRegistrar kGemmRegistrar;
@@ -1022,13 +943,22 @@ const GemmVariant* find_gemm(int format, const mb_gemm_config* config) {
   return nullptr;
 }
 
-// The launcher (and its registered name) a call will use: the variant's fast
-// kernel when the shape divides its tile and meets the path's rule, else its
-// checked kernel.
+// Estimated microseconds of a launch (see GemmCost): whole rounds of
+// 256 * resident tiles, then the rest.
+double gemm_cost(const GemmKernel& kernel, uint64_t m, uint64_t n, uint64_t steps) {
+  const uint64_t tiles = ((m + kernel.tile_m - 1) / kernel.tile_m) * ((n + kernel.tile_n - 1) / kernel.tile_n);
+  const uint64_t round = 256ull * kernel.resident;
+  const GemmCost& cost = kernel.cost;
+  auto one = [&](double filled) { return cost.tile + steps * (cost.step_empty + (cost.step_full - cost.step_empty) * filled); };
+  double total = (tiles / round) * one(1.0);
+  if (tiles % round) total += one(static_cast<double>(tiles % round) / round);
+  return total;
+}
+
+// The kernel a call will use.
 struct GemmChoice {
   const GemmVariant* variant;
-  GemmLauncher launch;
-  const char* name;
+  const GemmKernel* kernel;
 };
 
 int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k, const void* scale_a,
@@ -1050,21 +980,42 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
   // The tile count of the smallest tile any launcher uses bounds the grid.
   const uint64_t max_tiles = static_cast<uint64_t>((m + 63) / 64) * ((n + 63) / 64);
   if (max_tiles > 0x7fffffffull) return fail(MB_ERR_INVALID, "%s: too many tiles", entry);
-  const uint64_t row_bytes = row_bits / 8, steps = row_bytes / 128;
+  const uint64_t row_bytes = row_bits / 8, steps = (row_bytes + 127) / 128;
   const mb_gemm_config& v = variant->config;
-  bool fast = m % v.tile_m == 0 && n % v.tile_n == 0 && k % v.tile_k == 0;
-  // The staged kernel addresses each tile's operand rows (and the MXFP4 scale
-  // blocks) with 32-bit offsets in 128-byte K steps, runs an even number of
-  // at least four steps and moves scale rows with 16-byte DMAs.
-  if (variant->path == kStagedPath) {
-    fast = fast && row_bytes % 128 == 0 && 256 * row_bytes <= 0x7fffffffull && steps >= 4 && steps % 2 == 0;
-    if (format == MB_MATRIX_MXFP4)
-      fast = fast && aligned(scale_a, 16) && aligned(scale_b, 16) &&
-             steps * (m > n ? m : n) * 8 <= 0x7fffffffull;
-  }
+
+  const GemmKernel* best = nullptr;
+  double best_cost = 0;
+  auto consider = [&](const GemmKernel& kernel) {
+    if (kernel.format != format || kernel.tile_m > static_cast<int>(v.tile_m) ||
+        kernel.tile_n > static_cast<int>(v.tile_n))
+      return;
+    const double cost = gemm_cost(kernel, m, n, steps);
+    if (best == nullptr || cost < best_cost) best = &kernel, best_cost = cost;
+  };
+  // Both families address a tile's operand rows and the MXFP4 scale blocks
+  // with 32-bit offsets.
+  constexpr uint64_t kLimit = 0x7fffffff;
+  const bool scales_fit = format != MB_MATRIX_MXFP4 || steps * (m > n ? m : n) * 8 <= kLimit;
+  // The exact-shape kernels run an even number of at least four whole steps and
+  // move scale rows with 16-byte DMAs.
+  for (const GemmKernel& kernel : kExactKernels)
+    if (m % kernel.tile_m == 0 && n % kernel.tile_n == 0 && row_bytes % 128 == 0 && steps >= 4 && steps % 2 == 0 &&
+        256 * row_bytes <= kLimit && scales_fit &&
+        (format != MB_MATRIX_MXFP4 || (aligned(scale_a, 16) && aligned(scale_b, 16))))
+      consider(kernel);
+  // The ring kernels take every shape; their DMAs need dword-aligned scales,
+  // and their stores address a tile's rows of C with 32-bit offsets too.
+  int ring_count = 0;
+  const GemmKernel* ring = ring_kernels(&ring_count);
+  for (int i = 0; i < ring_count; ++i)
+    if (ring[i].tile_m * row_bytes <= kLimit && ring[i].tile_m * static_cast<uint64_t>(n) * variant->out_bytes <= kLimit &&
+        scales_fit && (format != MB_MATRIX_MXFP4 || (aligned(scale_a, 4) && aligned(scale_b, 4))))
+      consider(ring[i]);
+  if (best == nullptr)
+    for (const GemmKernel& kernel : kCheckedKernels)
+      if (kernel.format == format) best = &kernel;
   out->variant = variant;
-  out->launch = fast ? variant->launch : variant->launch_checked;
-  out->name = fast ? variant->name : variant->checked_name;
+  out->kernel = best;
   return MB_OK;
 }
 
@@ -1118,18 +1069,18 @@ int mb_gemm(int format, const mb_gemm_config* config, const void* a, uint64_t a_
   // tile count (group x tile columns) then stays within the int grid.
   const uint32_t max_group = (m + 63) / 64;
   const int group = static_cast<int>(group_m ? (group_m < max_group ? group_m : max_group)
-                                             : static_cast<uint32_t>(variant->default_group));
-  choice.launch(static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b), static_cast<const uint8_t*>(scale_a),
+                                             : static_cast<uint32_t>(choice.kernel->default_group));
+  choice.kernel->launch(static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b), static_cast<const uint8_t*>(scale_a),
                 static_cast<const uint8_t*>(scale_b), c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
                 group, static_cast<hipStream_t>(stream));
-  return launch_status(choice.name);
+  return launch_status(choice.kernel->name);
 }
 
 const char* mb_gemm_launched_kernel(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k,
                                     const void* scale_a, const void* scale_b) {
   mb::GemmChoice choice;
   if (mb::choose_gemm(format, config, m, n, k, scale_a, scale_b, "mb_gemm_launched_kernel", &choice)) return nullptr;
-  return choice.name;
+  return choice.kernel->name;
 }
 
 }  // extern "C"

@@ -1,0 +1,66 @@
+// Pieces shared by the GEMM kernels that stage their operands through LDS with
+// LDS-DMA loads (mb_gemm.hip, mb_gemm_ring.h).
+#pragma once
+
+#include <cstdint>
+#include <type_traits>
+
+#include "mb_internal.h"
+#include "mb_mfma.h"
+
+namespace mb {
+
+constexpr int kXcds = 8;
+
+// One 16-byte-per-lane LDS DMA: lane l's 16 bytes land at lds_addr + 16 * l.
+// Issued as inline assembly so the compiler's wait-count pass does not force a
+// full vmcnt(0) before every LDS read; the staged kernel issues it ahead of
+// compiler-visible loads, whose in-order vmcnt waits then cover it.
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset, uint32_t lds_addr) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(rsrc), "s"(soffset),
+               "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr))
+               : "memory");
+}
+
+// Word 3 of a gfx9 buffer resource: 32-bit data format, no swizzle, raw offsets.
+constexpr int kBufferWord3 = 0x00020000;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const uint8_t* base, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, bytes, kBufferWord3);
+}
+
+// Tile (tile_m, tile_n) of workgroup blockIdx.x: XCD-first numbering, then
+// GROUP_M-row bands (see the file comment).
+__device__ __forceinline__ void band_tile(int tiles_m, int tiles_n, int group_m, int& tile_m, int& tile_n) {
+  const int count = gridDim.x;
+  int pid = blockIdx.x;
+  if (count % kXcds == 0) pid = (pid % kXcds) * (count / kXcds) + pid / kXcds;
+  const int band = group_m * tiles_n;
+  const int first_m = (pid / band) * group_m;
+  const int rows_in_band = min(tiles_m - first_m, group_m);
+  tile_m = first_m + (pid % band) % rows_in_band;
+  tile_n = (pid % band) / rows_in_band;
+}
+
+// s_waitcnt's immediate for vmcnt(n) alone (n < 64): vmcnt's low four bits
+// at 3:0 and high two at 15:14, expcnt (6:4) and lgkmcnt (11:8) at their
+// maxima, which wait for nothing.
+constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+
+// Barrier that orders LDS only: global loads in flight stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// f(integral_constant<I>) for I = I0 .. N-1, so counts derived from I are constants.
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+}  // namespace mb

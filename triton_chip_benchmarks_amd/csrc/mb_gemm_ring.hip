@@ -1,0 +1,55 @@
+// The ring GEMM kernels of every format (see mb_gemm_ring.h).
+#include "mb_gemm_ring.h"
+
+#include "mb_gemm_host.h"
+
+namespace mb {
+namespace {
+
+template <class Op, int BM, int BN, int STAGES>
+void launch_ring(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m, int n,
+                 int k, int group_m, hipStream_t stream) {
+  gemm_ring_kernel<Op, BM, BN, STAGES><<<dim3(tile_count(m, n, BM, BN)), dim3(256), 0, stream>>>(
+      a, b, sa, sb, static_cast<typename Op::Out*>(c), m, n, k, group_m);
+}
+
+#define MB_RING(FMT, OP, BM, BN, STAGES, RESIDENT, COST, NAME)                                           \
+  GemmKernel {                                                                                           \
+    FMT, BM, BN, 8, RESIDENT, COST, NAME, reinterpret_cast<const void*>(gemm_ring_kernel<OP, BM, BN, STAGES>), \
+        launch_ring<OP, BM, BN, STAGES>                                                                  \
+  }
+#define MB_RING_SET(FMT, OP, TYPE, BK)                                                          \
+  MB_RING(FMT, OP, 256, 128, 3, 1, kCost256x128, "gemm_" TYPE "_256x128x" BK),                 \
+      MB_RING(FMT, OP, 128, 128, 4, 1, kCost128, "gemm_" TYPE "_128x128x" BK),             \
+      MB_RING(FMT, OP, 128, 128, 2, 2, kCost128Pair, "gemm_" TYPE "_128x128x" BK "_pair"),     \
+      MB_RING(FMT, OP, 64, 64, 3, 3, kCost64, "gemm_" TYPE "_64x64x" BK)
+
+const GemmKernel kRingKernels[] = {
+    MB_RING_SET(MB_MATRIX_BF16, MfmaBf16, "bf16", "64"),
+    MB_RING_SET(MB_MATRIX_F16, MfmaF16, "f16", "64"),
+    MB_RING_SET(MB_MATRIX_FP8_E4M3, MfmaFp8, "fp8", "128"),
+    MB_RING_SET(MB_MATRIX_I8, MfmaI8, "i8", "128"),
+    MB_RING_SET(MB_MATRIX_MXFP4, MfmaMxfp4, "mxfp4", "256"),
+    // FP32 and FP64 are bound by the matrix cores at every tile: no 256x128.
+    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 4, 1, kCostF32x128, "gemm_f32_128x128x32"),
+    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 2, 2, kCostF32x128Pair, "gemm_f32_128x128x32_pair"),
+    MB_RING(MB_MATRIX_F32, MfmaF32, 64, 64, 3, 3, kCostF32x64, "gemm_f32_64x64x32"),
+    MB_RING(MB_MATRIX_F64, MfmaF64, 128, 128, 4, 1, kCostF64x128, "gemm_f64_128x128x16"),
+    MB_RING(MB_MATRIX_F64, MfmaF64, 64, 64, 3, 3, kCostF64x64, "gemm_f64_64x64x16"),
+};
+
+struct RingRegistrar {
+  RingRegistrar() {
+    for (const GemmKernel& kernel : kRingKernels) register_kernel(kernel.name, kernel.kernel);
+  }
+};
+const RingRegistrar kRingRegistrar;
+
+}  // namespace
+
+const GemmKernel* ring_kernels(int* count) {
+  *count = static_cast<int>(sizeof(kRingKernels) / sizeof(kRingKernels[0]));
+  return kRingKernels;
+}
+
+}  // namespace mb
