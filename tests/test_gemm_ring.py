@@ -1,7 +1,7 @@
-"""The ring GEMM kernels at the edges of their tiles, K steps and dispatch, against oracle.tensor.
+"""The GEMM kernels of any shape (the ring and the ragged 256x256 ones) at the edges of their tiles, K steps and dispatch, against oracle.tensor.
 
 Operands are exact lattices (FP64: N(0,1) within its tolerance), so the
-comparison is exact. The shapes reach every ring kernel of every format with M
+comparison is exact. The shapes reach every such kernel of every format with M
 and N off its tile and K off its 128-byte step (a CPU test pins that).
 """
 
@@ -13,9 +13,9 @@ from test_gpu_gemm import FORMATS, _assert_matches, _configs, _run_gemm, _scale_
 
 CHUNK = {"bf16": 8, "fp16": 8, "fp32": 4, "fp64": 2, "int8": 16, "fp8": 16, "fp4": 32}  # elements per 16 bytes
 # (M, N, 16-byte chunks of K): one element, one step exactly, tails in M, N and K, odd and even step counts;
-# then one shape per larger ring tile.
+# then one shape per larger tile.
 SHAPES = [(1, 1, 1), (64, 64, 8), (65, 63, 9), (130, 70, 23), (192, 128, 16), (2040, 2035, 33), (2047, 2049, 9),
-          (2600, 2500, 161)]
+          (2600, 2500, 161), (3800, 3900, 161)]
 
 
 class _Scales:
@@ -39,16 +39,16 @@ def _launched(dtype, config, m, n, k):
 
 
 @pytest.mark.parametrize("dtype", FORMATS)
-def test_shapes_reach_every_ring_kernel(dtype):
+def test_shapes_reach_every_kernel_of_any_shape(dtype):
     from triton_chip_benchmarks_amd import _native
 
     prefix = _native.gemm_kernel_name(dtype, _configs(dtype)[0]).rsplit("_", 1)[0] + "_"
-    ring = {name for name in _native.kernel_names()
-            if name.startswith(prefix) and not name.endswith("_checked")
-            and "_256x256x" not in name and name != "gemm_f64_256x128x16"}
+    wanted = {name for name in _native.kernel_names()
+              if name.startswith(prefix) and not name.endswith("_checked")
+              and ("_256x256x" not in name or name.endswith("_ragged")) and name != "gemm_f64_256x128x16"}
     seen = {_launched(dtype, config, m, n, chunks * CHUNK[dtype])
             for config in _configs(dtype) for m, n, chunks in SHAPES}
-    assert ring <= seen, ring - seen
+    assert wanted <= seen, wanted - seen
 
 
 @pytest.mark.parametrize("dtype", FORMATS)
@@ -66,7 +66,7 @@ def test_a_launch_never_exceeds_the_requested_tile(dtype):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", FORMATS)
 @pytest.mark.parametrize("m,n,chunks", SHAPES)
-def test_ring_kernels_match_oracle(gpu, dtype, m, n, chunks):
+def test_kernels_of_any_shape_match_oracle(gpu, dtype, m, n, chunks):
     k = chunks * CHUNK[dtype]
     rng = np.random.default_rng(m + n + k)
     for launched in sorted({_launched(dtype, config, m, n, k) for config in _configs(dtype)}):
@@ -78,7 +78,7 @@ def test_ring_kernels_match_oracle(gpu, dtype, m, n, chunks):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", FORMATS)
-def test_ring_kernels_write_only_c_and_read_nothing_past_their_operands(gpu, dtype):
+def test_kernels_of_any_shape_write_only_c_and_read_nothing_past_their_operands(gpu, dtype):
     """C with guard rows and NaN (INT8: -3) bytes after A, B and the scales: a load past an edge that reached
     a product would show in C, a store past one in the guard."""
     import torch

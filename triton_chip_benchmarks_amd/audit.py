@@ -30,7 +30,7 @@ _MFMA_FORMAT = {"MfmaBf16": "bf16", "MfmaF16": "f16", "MfmaI8": "i8", "MfmaFp8":
 _PEAK_RE = re.compile(r"tensor_peak_(?:tied_)?kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])E")
 _GEMM_RE = re.compile(r"gemm_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E")
 _GEMM_RING_RE = re.compile(r"gemm_ring_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)EE")
-_GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)EE")
+_GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)E(?:Lb([01])E)?E")
 _ELEM_BITS = {"bf16": 16, "f16": 16, "i8": 8, "fp8": 8, "mxfp4": 4, "f32": 32, "f64": 64}
 _COPY_RE = re.compile(r"copy_kernelI(Dv4_j|j|h)Li(\d+)ELi([012])E")
 _READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)Li(\d+)E")
@@ -64,7 +64,7 @@ def registered_name(symbol: str) -> str | None:
     match = _GEMM_STAGED_RE.search(symbol)
     if match:
         fmt = _MFMA_FORMAT[match.group(1).removesuffix("x16")]
-        return f"gemm_{fmt}_256x256x{128 * 8 // _ELEM_BITS[fmt]}"
+        return f"gemm_{fmt}_256x256x{128 * 8 // _ELEM_BITS[fmt]}{'_ragged' if match.group(2) == '1' else ''}"
     if "gemm_dma_f64_kernelI" in symbol:
         return "gemm_f64_256x128x16"
     match = _COPY_RE.search(symbol)

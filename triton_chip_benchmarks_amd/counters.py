@@ -131,7 +131,8 @@ def registered_name(demangled: str) -> str:
         return ring_name(*args)
     if family in ("gemm_staged_kernel", "gemm_dma_kernel"):
         name = _MFMA_FORMAT[args[0].removesuffix("x16")]
-        return f"gemm_{name}_256x256x{128 * 8 // _ELEM_BITS[name]}"
+        ragged = "_ragged" if args[1:] in (["true"], ["1"]) else ""
+        return f"gemm_{name}_256x256x{128 * 8 // _ELEM_BITS[name]}{ragged}"
     if family == "gemm_dma_f64_kernel":
         return "gemm_f64_256x128x16"
     if family == "copy_kernel":

@@ -27,6 +27,7 @@
 //     MFMAs, so no burst of memory instructions stalls the in-order MFMA issue;
 //     one barrier per step. The DMA kernels move A straight into LDS with
 //     LDS-DMA loads instead.
+//     A RAGGED instantiation of gemm_dma_kernel takes any shape.
 //   * gemm_ring_kernel (mb_gemm_ring.h): 64x64, 128x128 and 256x128 tiles, any
 //     shape. Large tiles leave CUs idle on small problems: 2048^3 in BF16 has
 //     64 tiles of 256x256 (39.3 us) but 256 of 128x128 (20.4 us).
@@ -486,7 +487,13 @@ __global__ void __launch_bounds__(256)
 // accumulators' zeroing from the first MFMA and the last MFMA from the
 // epilogue's reads. Every block update is its own scheduling region, so
 // program order is the issue order.
-template <class Op>
+//
+// RAGGED takes any shape, as the ring kernels do: DMAs and stores past M, N or
+// K get out-of-range offsets from the buffer bounds check, and an odd step
+// count is rounded up with a step of zeros. Its row offsets sit in registers
+// instead of the scalar offset, which the bounds check subtracts from the
+// buffer's size and must not exceed it.
+template <class Op, bool RAGGED>
 __global__ void __launch_bounds__(256)
     gemm_dma_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__,
                     const uint8_t* __restrict__, typename Op::Out* __restrict__ C, int M, int N, int K,
@@ -504,15 +511,21 @@ __global__ void __launch_bounds__(256)
   if (K < 0) lds[threadIdx.x] = 0;  // keeps DMA-written reads live; never executed
 
   int tile_m, tile_n;
-  band_tile(M / BM, N / BM, group_m, tile_m, tile_n);
+  if constexpr (RAGGED)
+    band_tile_any((static_cast<uint32_t>(M) + BM - 1) / BM, (static_cast<uint32_t>(N) + BM - 1) / BM, group_m, tile_m,
+                  tile_n);
+  else
+    band_tile(M / BM, N / BM, group_m, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BM;
   const int row_bytes = K * Op::ELEM_BITS / 8;
-  const int k_steps = row_bytes / ROWB, last = k_steps - 1;
+  const int k_steps = (row_bytes + ROWB - 1) / ROWB, last = k_steps - 1;
 
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(A + static_cast<int64_t>(m0) * row_bytes, BM * row_bytes);
-  const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(B + static_cast<int64_t>(n0) * row_bytes, BM * row_bytes);
+  const __amdgpu_buffer_rsrc_t ra =
+      buffer_rsrc(A + static_cast<int64_t>(m0) * row_bytes, (RAGGED ? min(BM, M - m0) : BM) * row_bytes);
+  const __amdgpu_buffer_rsrc_t rb =
+      buffer_rsrc(B + static_cast<int64_t>(n0) * row_bytes, (RAGGED ? min(BM, N - n0) : BM) * row_bytes);
   // Both operands: instruction i of wave w moves rows 64w+8i .. +7 (lane l row l/8, the chunk stored at
   // physical chunk l%8 of its row) into LDS region `region`: A slots are regions 0..2, B slots 3 and 4.
   const int drow = lane >> 3;
@@ -520,9 +533,23 @@ __global__ void __launch_bounds__(256)
   const int dvoff1 = drow * row_bytes + (((lane & 7) ^ ((drow >> 1) | 4)) << 4);
   const uint32_t lds_base =
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
+  // RAGGED: the whole row offset per instruction, and the step bytes below
+  // which the lane's chunk lies inside its row.
+  int dvoff[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) dvoff[i] = (64 * wave + 8 * i) * row_bytes + ((i & 1) ? dvoff1 : dvoff0);
+  const int limit0 = row_bytes - (((lane & 7) ^ (drow >> 1)) << 4);
+  const int limit1 = row_bytes - (((lane & 7) ^ ((drow >> 1) | 4)) << 4);
   auto dma = [&](__amdgpu_buffer_rsrc_t r, int region, int kt, int i) __attribute__((always_inline)) {
     const int row = 64 * wave + 8 * i;
-    dma16(r, (i & 1) ? dvoff1 : dvoff0, kt * ROWB + row * row_bytes, lds_base + region * REGION + row * ROWB);
+    const uint32_t to = lds_base + region * REGION + row * ROWB;
+    if constexpr (RAGGED) {
+      const int kb = kt * ROWB;
+      dma16(r, kb < ((i & 1) ? limit1 : limit0) ? dvoff[i] : kOutOfRange,
+            __builtin_amdgcn_readfirstlane(kt < k_steps ? kb : 0), to);
+    } else {
+      dma16(r, (i & 1) ? dvoff1 : dvoff0, min(kt, last) * ROWB + row * row_bytes, to);
+    }
   };
 
   const int wm = wave & 1, wn = wave >> 1;
@@ -566,11 +593,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dma(ra, p, min(p, last), i);
+    for (int i = 0; i < 8; ++i) dma(ra, p, p, i);
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dma(rb, 3 + p, min(p, last), i);
+    for (int i = 0; i < 8; ++i) dma(rb, 3 + p, p, i);
   __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
   lds_barrier();
 
@@ -598,7 +625,7 @@ __global__ void __launch_bounds__(256)
       constexpr int rd = q < 8 && q % 2 == 0 ? q / 2 : -1;
       if constexpr (rd >= 0) fb[rd] = frag_b(s, rd);
       constexpr int da = q % 4 == 1 ? q / 4 : -1;
-      if constexpr (da >= 0) dma(ra, prev_slot, min(kt + 2, last), da);
+      if constexpr (da >= 0) dma(ra, prev_slot, kt + 2, da);
       mma(fa[i], fb[j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -610,7 +637,7 @@ __global__ void __launch_bounds__(256)
       constexpr int rd = q < 8 && q % 2 == 0 ? 4 + q / 2 : -1;
       if constexpr (rd >= 0) fb[rd] = frag_b(s ^ 1, rd);
       constexpr int db = q % 4 == 1 ? q / 4 : -1;
-      if constexpr (db >= 0) dma(rb, 3 + s, min(kt + 2, last), db);
+      if constexpr (db >= 0) dma(rb, 3 + s, kt + 2, db);
       mma(fa[i], fb[j], acc[i][j]);
       if constexpr (j == 3) fa[i] = frag_a(next_slot, i);
       __builtin_amdgcn_sched_barrier(0);
@@ -626,6 +653,25 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int j = 0; j < TILES; ++j) acc_hazard_fence(acc[i][j]);
 
+  if constexpr (RAGGED) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    constexpr int ES = sizeof(typename Op::Out);
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+        C + static_cast<int64_t>(m0) * N + n0, (short)0, min(BM, M - m0) * N * ES - n0 * ES, kBufferWord3);
+#pragma unroll
+    for (int j = 0; j < TILES; ++j) {
+      const int col = wn * 128 + j * Op::N + lrow;
+      const bool inside = n0 + col < N;
+#pragma unroll
+      for (int i = 0; i < TILES; ++i)
+#pragma unroll
+        for (int r = 0; r < Op::ACC_REGS; ++r) {
+          const int offset = ((wm * 128 + i * Op::M + Op::out_row(lane, r)) * N + col) * ES;
+          const typename Op::Out value = acc[i][j][r];
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rc, inside ? offset : kOutOfRange, 0, 0);
+        }
+    }
+  } else {
 #pragma unroll
   for (int i = 0; i < TILES; ++i)
 #pragma unroll
@@ -636,6 +682,7 @@ __global__ void __launch_bounds__(256)
         const int col = n0 + wn * 128 + j * Op::N + lrow;
         C[static_cast<int64_t>(row) * N + col] = acc[i][j][r];
       }
+  }
 #endif
 }
 
@@ -839,7 +886,7 @@ constexpr auto exact_kernel_fn() {
   else if constexpr (Op::ELEM_BITS == 64)
     return gemm_dma_f64_kernel<Op>;
   else
-    return gemm_dma_kernel<Op>;
+    return gemm_dma_kernel<Op, false>;
 }
 
 // Tile width of the exact-shape kernel (its height is 256).
@@ -870,6 +917,27 @@ const GemmKernel kExactKernels[] = {
     MB_EXACT(MB_MATRIX_MXFP4, MfmaMxfp4, 8, kCost256, "gemm_mxfp4_256x256x256"),
     MB_EXACT(MB_MATRIX_F64, MfmaF64, 8, kCostF64x256, "gemm_f64_256x128x16"),
     MB_EXACT(MB_MATRIX_F32, MfmaF32x16, 8, kCostF32x256, "gemm_f32_256x256x32"),
+};
+
+template <class Op>
+void launch_ragged(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const uint8_t* sb, void* c, int m, int n,
+                   int k, int group_m, hipStream_t stream) {
+  gemm_dma_kernel<Op, true><<<dim3(tile_count(m, n, 256, 256)), dim3(256), 0, stream>>>(
+      a, b, sa, sb, static_cast<typename Op::Out*>(c), m, n, k, group_m);
+}
+
+// 256x256 tiles of any shape. Against the ring's 256x128 (us): FP8 5000x3000x4112
+// 60.9 and 73.2, BF16 4000^3 100.9 and 122.1, 8191x8191x8192 763 and 888 (8192^3
+// in exact tiles 700). FP32 gains nothing: 128x128 is as fast at 4000^3.
+#define MB_RAGGED(FMT, OP, GROUP, NAME)                                                                    \
+  GemmKernel {                                                                                                   \
+    FMT, 256, 256, GROUP, 1, kCost256, NAME, reinterpret_cast<const void*>(gemm_dma_kernel<OP, true>), launch_ragged<OP> \
+  }
+const GemmKernel kRaggedKernels[] = {
+    MB_RAGGED(MB_MATRIX_BF16, MfmaBf16x16, 4, "gemm_bf16_256x256x64_ragged"),
+    MB_RAGGED(MB_MATRIX_F16, MfmaF16x16, 4, "gemm_f16_256x256x64_ragged"),
+    MB_RAGGED(MB_MATRIX_FP8_E4M3, MfmaFp8x16, 6, "gemm_fp8_256x256x128_ragged"),
+    MB_RAGGED(MB_MATRIX_I8, MfmaI8x16, 7, "gemm_i8_256x256x128_ragged"),
 };
 
 // Any shape whose rows are too long for the ring kernels' 32-bit offsets.
@@ -928,6 +996,7 @@ const GemmVariant kGemmVariants[] = {
 struct GemmRegistrar {
   GemmRegistrar() {
     for (const GemmKernel& kernel : kExactKernels) register_kernel(kernel.name, kernel.kernel);
+    for (const GemmKernel& kernel : kRaggedKernels) register_kernel(kernel.name, kernel.kernel);
     for (const GemmKernel& kernel : kCheckedKernels) register_kernel(kernel.name, kernel.kernel);
   }
 };
@@ -1003,14 +1072,19 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
         256 * row_bytes <= kLimit && scales_fit &&
         (format != MB_MATRIX_MXFP4 || (aligned(scale_a, 16) && aligned(scale_b, 16))))
       consider(kernel);
-  // The ring kernels take every shape; their DMAs need dword-aligned scales,
-  // and their stores address a tile's rows of C with 32-bit offsets too.
+  // The ragged and ring kernels take every shape; the ring's scale DMAs need
+  // dword-aligned scales, and the stores address a tile's rows of C with 32-bit
+  // offsets too.
+  auto consider_any_shape = [&](const GemmKernel& kernel) {
+    if (kernel.tile_m * row_bytes <= kLimit &&
+        kernel.tile_m * static_cast<uint64_t>(n) * variant->out_bytes <= kLimit && scales_fit &&
+        (format != MB_MATRIX_MXFP4 || (aligned(scale_a, 4) && aligned(scale_b, 4))))
+      consider(kernel);
+  };
   int ring_count = 0;
   const GemmKernel* ring = ring_kernels(&ring_count);
-  for (int i = 0; i < ring_count; ++i)
-    if (ring[i].tile_m * row_bytes <= kLimit && ring[i].tile_m * static_cast<uint64_t>(n) * variant->out_bytes <= kLimit &&
-        scales_fit && (format != MB_MATRIX_MXFP4 || (aligned(scale_a, 4) && aligned(scale_b, 4))))
-      consider(ring[i]);
+  for (const GemmKernel& kernel : kRaggedKernels) consider_any_shape(kernel);
+  for (int i = 0; i < ring_count; ++i) consider_any_shape(ring[i]);
   if (best == nullptr)
     for (const GemmKernel& kernel : kCheckedKernels)
       if (kernel.format == format) best = &kernel;

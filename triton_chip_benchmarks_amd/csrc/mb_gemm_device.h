@@ -42,6 +42,22 @@ __device__ __forceinline__ void band_tile(int tiles_m, int tiles_n, int group_m,
   tile_n = (pid % band) / rows_in_band;
 }
 
+// A byte offset past every buffer resource (num_records stays below 2^31):
+// loads from it give zeros, stores to it are dropped.
+constexpr int kOutOfRange = static_cast<int>(0x80000000u);
+
+// Tile of workgroup blockIdx.x for any grid size: XCD x (ids x, x+8, ..) owns
+// a contiguous share of the band order, the first count % 8 XCDs one tile more.
+__device__ __forceinline__ void band_tile_any(int tiles_m, int tiles_n, int group_m, int& tile_m, int& tile_n) {
+  const int count = gridDim.x, xcd = blockIdx.x % kXcds, index = blockIdx.x / kXcds;
+  const int pid = xcd * (count / kXcds) + min(xcd, count % kXcds) + index;
+  const int band = group_m * tiles_n;
+  const int first_m = (pid / band) * group_m;
+  const int rows_in_band = min(tiles_m - first_m, group_m);
+  tile_m = first_m + (pid % band) % rows_in_band;
+  tile_n = (pid % band) / rows_in_band;
+}
+
 // s_waitcnt's immediate for vmcnt(n) alone (n < 64): vmcnt's low four bits
 // at 3:0 and high two at 15:14, expcnt (6:4) and lgkmcnt (11:8) at their
 // maxima, which wait for nothing.

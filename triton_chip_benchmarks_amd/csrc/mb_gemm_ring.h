@@ -6,22 +6,6 @@
 
 namespace mb {
 
-// A byte offset past every buffer resource (num_records stays below 2^31):
-// loads from it give zeros, stores to it are dropped.
-constexpr int kOutOfRange = static_cast<int>(0x80000000u);
-
-// Tile of workgroup blockIdx.x for any grid size: XCD x (ids x, x+8, ..) owns
-// a contiguous share of the band order, the first count % 8 XCDs one tile more.
-__device__ __forceinline__ void band_tile_any(int tiles_m, int tiles_n, int group_m, int& tile_m, int& tile_n) {
-  const int count = gridDim.x, xcd = blockIdx.x % kXcds, index = blockIdx.x / kXcds;
-  const int pid = xcd * (count / kXcds) + min(xcd, count % kXcds) + index;
-  const int band = group_m * tiles_n;
-  const int first_m = (pid / band) * group_m;
-  const int rows_in_band = min(tiles_m - first_m, group_m);
-  tile_m = first_m + (pid % band) % rows_in_band;
-  tile_n = (pid % band) / rows_in_band;
-}
-
 template <class Op, int BM, int BN, int STAGES>
 struct RingTile {
   static constexpr int ROWB = 128;                     // bytes of K per row and step
@@ -76,7 +60,7 @@ struct RingTile {
 //
 // Measured against the largest tile it replaces (us): BF16 256^3 10.6 -> 3.1,
 // 1024^3 22.3 -> 5.6, 2048^3 39.3 -> 20.4, 2560^3 47.9 -> 34.1; FP16
-// 1000x744x1000 16.8 -> 5.5; FP8 5000x3000x4112 88 -> 73; MXFP4 2048^3
+// 1000x744x1000 16.8 -> 5.5; MXFP4 2048^3
 // 19.4 -> 10.2; FP32 1024^3 226 -> 22; FP64 2048^3 456 -> 248.
 //
 // Any shape: rows past M or N, chunks past K and steps past the last get an
