@@ -255,7 +255,7 @@ class CopyWorkload(Workload):
         bb.check_fill(self.dst)
         bound = bb.rw_bound(rates["read"], rates["write"])
         return {"read_only_gbps": rates["read"], "write_only_gbps": rates["write"], "rw_bound_gbps": bound,
-                "read_config": dict(r, kernel="read_sum_fp32_vec"), "write_config": dict(w, kernel="fill_dwordx4_stream"),
+                "read_config": dict(r, kernel=bb.read_kernel("fp32", r["block_elements"])), "write_config": dict(w, kernel="fill_dwordx4_stream"),
                 "launches_per_leg": BOUND_LAUNCHES,
                 "method": "read-only (mb_read_sum) and write-only (mb_fill) streams over the copy's own 1 GiB buffers, "
                           "both validated; bound = harmonic mean of the two rates"}

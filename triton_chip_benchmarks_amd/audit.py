@@ -34,6 +34,7 @@ _GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)E(?:Lb
 _ELEM_BITS = {"bf16": 16, "f16": 16, "i8": 8, "fp8": 8, "mxfp4": 4, "f32": 32, "f64": 64}
 _COPY_RE = re.compile(r"copy_kernelI(Dv4_j|j|h)Li(\d+)ELi([012])E")
 _READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)Li(\d+)E")
+_READ_PACKED_RE = re.compile(r"read_sum_packed_kernelI(f|DF16_|t)Li(\d+)E")
 _VECTOR_RE = re.compile(r"vector_(\w+?)_kernelILi(\d+)E")
 _COPY_UNIT = {"Dv4_j": "dwordx4", "j": "dword", "h": "byte"}
 _READ_TYPE = {"f": "f32", "DF16_": "f16", "t": "bf16"}
@@ -71,10 +72,13 @@ def registered_name(symbol: str) -> str | None:
     if match:
         unit, vpt, policy = match.groups()
         return f"copy_{_COPY_UNIT[unit]}_vpt{vpt}{('', '_nt', '_stream')[int(policy)]}"
+    match = _READ_PACKED_RE.search(symbol)
+    if match:
+        dtype, vectors = match.groups()
+        return f"read_sum_{_READ_TYPE[dtype]}_packed{vectors}"
     match = _READ_RE.search(symbol)
     if match:
-        dtype, vec = match.groups()
-        return f"read_sum_{_READ_TYPE[dtype]}{'_vec' if vec != '1' else ''}"
+        return f"read_sum_{_READ_TYPE[match.group(1)]}_vec"
     match = _VECTOR_RE.search(symbol)
     if match:
         kind, unroll = match.groups()

@@ -99,6 +99,12 @@ def rw_bound(read_gbps, write_gbps):
     return 2.0 / (1.0 / read_gbps + 1.0 / write_gbps)
 
 
+def read_kernel(dtype, block_size):
+    """Registered name of the kernel mb_read_sum launches: blocks of up to 256 16-byte vectors share a wave."""
+    vectors = block_size * (4 if dtype == "fp32" else 2) // VECTOR_BYTES
+    return f"read_sum_{dtype.replace('fp', 'f')}_{f'packed{vectors}' if vectors <= 256 else 'vec'}"
+
+
 def launch_read(src, sink, block_size, block_threads):
     """sink[i] <- sum of src block i, through mb_read_sum."""
     segments = -(-src.numel() // block_size)
@@ -303,7 +309,7 @@ def main(argv=None):
                         run()
                         correctness = check_read(src, sink, block)
                         write_bytes = sink.numel() * sink.element_size()
-                        kernel = f"read_sum_{args.dtype}_vec"
+                        kernel = read_kernel(args.dtype, block)
                     timings = measure(run, args)
                     traffic = write_bytes if mode == "write" else buffer_bytes + write_bytes
                     gbps = traffic / (timings["median_ms"] * 1e6)

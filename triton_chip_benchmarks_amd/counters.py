@@ -139,9 +139,9 @@ def registered_name(demangled: str) -> str:
         unit = "dwordx4" if "__vector(4)" in args[0] else "byte" if "char" in args[0] else "dword"
         policy = {"0": "", "false": "", "1": "_nt", "true": "_nt", "2": "_stream"}[args[2]]
         return f"copy_{unit}_vpt{args[1]}{policy}"
-    if family == "read_sum_kernel":
-        kind = {"float": "f32", "_Float16": "f16", "__bf16": "bf16"}.get(args[0], args[0])
-        return f"read_sum_{kind}{'_vec' if args[1] != '1' else ''}"
+    if family in ("read_sum_kernel", "read_sum_packed_kernel"):
+        kind = {"float": "f32", "_Float16": "f16", "__bf16": "bf16", "unsigned short": "bf16"}.get(args[0], args[0])
+        return f"read_sum_{kind}_{'vec' if family == 'read_sum_kernel' else 'packed' + args[1]}"
     if family == "fill_kernel":
         return "fill_dwordx4" + {"0": "", "1": "_nt", "2": "_stream"}.get(args[0], "")
     if family.startswith("vector_") and family.endswith("_kernel"):

@@ -9,14 +9,13 @@
 // XCD's L2 instead of leaving dirty lines to be evicted later) - on MI355X the
 // last measures ~1% faster than nt stores for HBM-sized copies.
 //
-// Read: one wave reduces one segment of `block_elements` values to a single
-// float (the reference's per-program sum), streaming it with non-temporal
-// 16-byte loads (eight in flight per lane) into eight independent
-// accumulators, then a butterfly across the 64 lanes. Non-temporal loads
-// stream HBM ~7% faster than plain ones on MI355X (88-90% of 8 TB/s against
-// 82-84%, read-only). The
-// summation depth stays below the 2*eps*log2(block) bound the reference
-// validates block sums with (bench_bandwidth.py:87).
+// Read: a wave streams its segments of `block_elements` values with
+// non-temporal 16-byte loads and reduces each to a single float (the
+// reference's per-program sum): one segment of more than 4 KiB, or several that
+// fill 4 KiB. Non-temporal loads stream HBM ~7% faster than plain ones on
+// MI355X (88-90% of 8 TB/s against 82-84%, read-only). The summation depth
+// stays below the 2*eps*log2(block) bound the reference validates block sums
+// with (bench_bandwidth.py:87).
 #include "mb_internal.h"
 
 namespace mb {
@@ -141,12 +140,151 @@ __device__ __forceinline__ float wave_sum(float value) {
   return value;
 }
 
-// One wave per segment; waves stride over the segments of the buffer.
-// VEC elements per lane per load (16 bytes, or 1 for unaligned sources).
+// 16 bytes at any address: gfx950 takes a global_load_dwordx4 there.
+typedef u32x4 u32x4_unaligned __attribute__((aligned(1)));
+
+template <typename T>
+__device__ __forceinline__ u32x4 load_vector(const T* ptr) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_unaligned*>(ptr));
+}
+
+// value[j] = the sum of the 16 bytes at ptr + j * 64 vectors, for N loads: all
+// of them in flight before any is summed, or, `serial`, one after the other.
+template <typename T, int N>
+__device__ __forceinline__ void load_and_sum(float (&value)[N], const T* ptr, bool serial) {
+  constexpr int VEC = 16 / sizeof(T);
+  if (serial) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      value[j] = vector_sum<T, VEC>(load_vector(ptr + j * 64 * VEC));
+      asm volatile("" : "+v"(ptr) : "v"(value[j]));  // the next address waits for this sum
+    }
+  } else {
+    u32x4 raw[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) raw[j] = load_vector(ptr + j * 64 * VEC);
+#pragma unroll
+    for (int j = 0; j < N; ++j) value[j] = vector_sum<T, VEC>(raw[j]);
+  }
+}
+
+// The sum of `count` elements by one wave, eight bounded loads in flight: the
+// buffer's clipped last segment.
+template <typename T>
+__device__ __forceinline__ float clipped_sum(const T* base, uint32_t count, uint32_t lane) {
+  constexpr int VEC = 16 / sizeof(T);
+  const uint32_t vectors = count / VEC;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (uint32_t p = lane; p < vectors; p += 512) {
+    u32x4 raw[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j)
+      raw[j] = p + j * 64 < vectors ? load_vector(base + (p + j * 64) * VEC) : u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += vector_sum<T, VEC>(raw[j]);
+  }
+  if (lane < count % VEC) acc[0] += to_float(base[vectors * VEC + lane]);
+  return wave_sum(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
+}
+
+// 16-byte vectors a wave of the packed read sums.
+constexpr uint32_t kPackedVectors = 256;
+
+// Segments of V 16-byte vectors, V from 8 to kPackedVectors: one wave sums the
+// segments of 4 KiB.
+//
+// Bound by HBM: 1 GiB takes 150-160 us (6.7-7.2 TB/s) at every block size.
+// One wave per segment, as larger blocks have it, starts and folds a wave for
+// 1 KiB at FP32 blocks of 256 (220 us) and reads two bytes per lane where a
+// segment is shorter than a wave's load (BF16 blocks of 256: 721 us). Here a
+// lane's loads of one segment are summed first; then the values of different
+// segments fold over the lanes together: at offset o, two values become one, a
+// lane with bit o clear keeping the first and adding its partner's share of it,
+// the others the second. That takes half the shuffles of such a step away and
+// leaves each sum in the lanes that store it. Adding commutes, so a sum's tree
+// is the plain butterfly's.
+//
+// The four loads go out together where waves are few (FP32 blocks of 1024,
+// 8 MiB: 4.9 us, one by one 6.3; 256 MiB, 64-value blocks: 40.6 and 44.8) and
+// from unaligned sources (1 GiB of FP32 156 and 162). Past 131072 waves (half a
+// GiB here), one load per wave at a time covers the latency (32 waves of 1 KiB
+// per CU) and more only disturbs the DRAM pages: 1 GiB takes 146 us one by one
+// and 157 together.
+template <typename T, int V>
+__global__ void __launch_bounds__(1024)
+    read_sum_packed_kernel(const T* __restrict__ src, float* __restrict__ sink, uint64_t elements, uint64_t chunks,
+                           bool serial) {
+  constexpr int VEC = 16 / sizeof(T), LOADS = kPackedVectors / 64;
+  constexpr int PER_SEGMENT = V > 64 ? V / 64 : 1;       // loads of one segment
+  constexpr int VALUES = LOADS / PER_SEGMENT;            // segments a lane has a share of
+  constexpr int LANES = V < 64 ? V : 64;                 // lanes sharing a segment
+  constexpr uint32_t SEGMENTS = LOADS * 64 / V;          // of one chunk
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t waves_per_block = blockDim.x >> 6;
+  const uint64_t whole = elements / (V * VEC);  // segments that are not clipped
+  const uint64_t total_waves = static_cast<uint64_t>(gridDim.x) * waves_per_block;
+  for (uint64_t chunk = blockIdx.x * waves_per_block + (threadIdx.x >> 6); chunk <= chunks; chunk += total_waves) {
+    if (chunk == chunks) {  // after the last chunk of whole segments: the clipped one
+      const uint32_t left = static_cast<uint32_t>(elements - whole * (V * VEC));
+      if (left) {
+        const float total = clipped_sum(src + whole * (V * VEC), left, lane);
+        if (lane == 0) sink[whole] = total;
+      }
+      break;
+    }
+    const uint64_t first = chunk * SEGMENTS;
+    const T* base = src + chunk * (LOADS * 64 * VEC) + lane * VEC;
+    float value[LOADS];
+    if (first + SEGMENTS <= whole) {
+      load_and_sum(value, base, serial);
+    } else {
+      const uint32_t vectors = static_cast<uint32_t>(whole - first) * V;
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j)
+        value[j] = j * 64 + lane < vectors ? vector_sum<T, VEC>(load_vector(base + j * 64 * VEC)) : 0.f;
+    }
+    // One value per segment: pairwise over its loads.
+#pragma unroll
+    for (int width = 1; width < PER_SEGMENT; width *= 2)
+#pragma unroll
+      for (int j = 0; j < LOADS; j += 2 * width) value[j] += value[j + width];
+#pragma unroll
+    for (int i = 1; i < VALUES; ++i) value[i] = value[i * PER_SEGMENT];
+    int values = VALUES, index = 0;
+#pragma unroll
+    for (int offset = LANES / 2; offset > 0; offset >>= 1) {
+      if (values > 1) {
+        const bool second = lane & offset;
+#pragma unroll
+        for (int i = 0; i < values / 2; ++i) {
+          const float keep = second ? value[2 * i + 1] : value[2 * i];
+          const float give = second ? value[2 * i] : value[2 * i + 1];
+          value[i] = keep + __shfl_xor(give, offset, 64);
+        }
+        index += second ? VALUES / values : 0;  // bit 0 of the value's number first
+        values /= 2;
+      } else {
+        value[0] += __shfl_xor(value[0], offset, 64);
+      }
+    }
+    // Lanes whose plain-butterfly bits are clear hold one segment each (several
+    // values in every lane where the lanes ran out first).
+    constexpr int MERGES = VALUES == 4 ? 2 : VALUES == 2 ? 1 : 0;
+    constexpr int STEPS = LANES == 64 ? 6 : LANES == 32 ? 5 : LANES == 16 ? 4 : 3;
+    static_assert(MERGES <= STEPS, "every value folds away");
+    constexpr uint32_t PLAIN = (1u << (STEPS - MERGES)) - 1;
+    const uint64_t segment = first + index * (64 / LANES) + lane / LANES;
+    if ((lane & PLAIN) == 0 && segment < whole) sink[segment] = value[0] + 0.f;
+  }
+}
+
+// Segments of more than kPackedVectors 16-byte vectors: one wave per segment; waves stride
+// over the segments of the buffer.
 template <typename T, int VEC>
 __global__ void __launch_bounds__(1024) read_sum_kernel(const T* __restrict__ src, float* __restrict__ sink,
                                                          uint64_t elements, uint32_t block_elements,
-                                                         uint64_t segments) {
+                                                         uint64_t segments, bool serial) {
+  static_assert(VEC * sizeof(T) == 16, "16-byte loads");
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t waves_per_block = blockDim.x >> 6;
   const uint64_t wave = blockIdx.x * waves_per_block + (threadIdx.x >> 6);
@@ -154,36 +292,22 @@ __global__ void __launch_bounds__(1024) read_sum_kernel(const T* __restrict__ sr
   const uint32_t chunk = 64 * VEC;  // elements one wave covers per load
   for (uint64_t segment = wave; segment < segments; segment += total_waves) {
     const uint64_t first = segment * block_elements;
-    const uint64_t count = (elements - first < block_elements) ? elements - first : block_elements;
     const T* base = src + first;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (count == block_elements && block_elements >= chunk) {
+    float total;
+    if (elements - first >= block_elements) {
+      // Load p feeds acc[p & 7]; block_elements is a multiple of eight loads.
+      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       const uint32_t loads = block_elements / chunk;
-      if constexpr (VEC > 1) {
-        // Vector path: eight 16-byte loads in flight per lane before any is
-        // summed (load p still feeds acc[p & 7], in the same order). Segments
-        // of fewer than eight loads take the remainder loop only.
-        uint32_t p = 0;
-        for (; p + 8 <= loads; p += 8) {
-          u32x4 raw[8];
+      for (uint32_t p = 0; p < loads; p += 8) {
+        float value[8];
+        load_and_sum(value, base + p * chunk + lane * VEC, serial);
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + (p + j) * chunk + lane * VEC));
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[j] += vector_sum<T, VEC>(raw[j]);
-        }
-        for (; p < loads; ++p)
-          acc[p & 7] += vector_sum<T, VEC>(
-              __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(base + p * chunk + lane * VEC)));
-      } else {
-        for (uint32_t p = 0; p < loads; ++p) acc[p & 7] += to_float(base[p * chunk + lane]);
+        for (int j = 0; j < 8; ++j) acc[j] += value[j];
       }
+      total = wave_sum(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
     } else {
-      // Clipped last segment, or a segment narrower than one vector load.
-      for (uint64_t i = lane; i < count; i += 64) acc[(i >> 6) & 7] += to_float(base[i]);
+      total = clipped_sum(base, static_cast<uint32_t>(elements - first), lane);
     }
-    const float total =
-        wave_sum(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
     if (lane == 0) sink[segment] = total;
   }
 }
@@ -232,28 +356,47 @@ MB_REGISTER_KERNEL("fill_dwordx4_nt", (fill_kernel<kNontemporal>));
 MB_REGISTER_KERNEL("fill_dwordx4_stream", (fill_kernel<kStream>));
 MB_REGISTER_KERNEL("fill_tail", fill_tail_kernel);
 MB_REGISTER_KERNEL("read_sum_f32_vec", (read_sum_kernel<float, 4>));
-MB_REGISTER_KERNEL("read_sum_f32", (read_sum_kernel<float, 1>));
 MB_REGISTER_KERNEL("read_sum_f16_vec", (read_sum_kernel<_Float16, 8>));
-MB_REGISTER_KERNEL("read_sum_f16", (read_sum_kernel<_Float16, 1>));
 MB_REGISTER_KERNEL("read_sum_bf16_vec", (read_sum_kernel<uint16_t, 8>));
-MB_REGISTER_KERNEL("read_sum_bf16", (read_sum_kernel<uint16_t, 1>));
+#define MB_REGISTER_READ_PACKED(T, TNAME)                                            \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed8", (read_sum_packed_kernel<T, 8>));     \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed16", (read_sum_packed_kernel<T, 16>));   \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed32", (read_sum_packed_kernel<T, 32>));   \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed64", (read_sum_packed_kernel<T, 64>));   \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed128", (read_sum_packed_kernel<T, 128>)); \
+  MB_REGISTER_KERNEL("read_sum_" TNAME "_packed256", (read_sum_packed_kernel<T, 256>))
+MB_REGISTER_READ_PACKED(float, "f32");
+MB_REGISTER_READ_PACKED(_Float16, "f16");
+MB_REGISTER_READ_PACKED(uint16_t, "bf16");
 
 template <typename T>
 int launch_read(const void* src, float* sink, uint64_t elements, uint32_t block_elements, uint32_t threads,
                 hipStream_t stream) {
-  constexpr int kVec = 16 / sizeof(T);
-  const uint64_t segments = (elements + block_elements - 1) / block_elements;
+  constexpr uint32_t kVec = 16 / sizeof(T);
+  const uint64_t segments = elements / block_elements + (elements % block_elements != 0);
+  const uint64_t whole = elements / block_elements;
   const uint64_t waves_per_block = threads / 64;
-  uint64_t grid = (segments + waves_per_block - 1) / waves_per_block;
-  // Waves stride over segments, so a bounded grid still covers every segment.
+  const uint32_t vectors = block_elements / kVec;
+  // Waves: one per 4 KiB of whole segments and one for a clipped segment, or
+  // one per segment. They stride, so a bounded grid still covers everything.
+  const bool packed = vectors <= kPackedVectors;
+  const uint64_t per_chunk = packed ? kPackedVectors / vectors : 1;
+  const uint64_t chunks = (whole + per_chunk - 1) / per_chunk;
+  const uint64_t waves = packed ? chunks + (segments != whole) : segments;
+  uint64_t grid = (waves + waves_per_block - 1) / waves_per_block;
+  const bool serial = waves > 131072 && aligned(src, 16);  // see read_sum_packed_kernel
   const uint64_t max_grid = 1ull << 20;
   if (grid > max_grid) grid = max_grid;
   const T* s = static_cast<const T*>(src);
   dim3 g(static_cast<uint32_t>(grid)), b(threads);
-  if (aligned(src, 16) && block_elements >= 64u * kVec) {
-    read_sum_kernel<T, kVec><<<g, b, 0, stream>>>(s, sink, elements, block_elements, segments);
-  } else {
-    read_sum_kernel<T, 1><<<g, b, 0, stream>>>(s, sink, elements, block_elements, segments);
+  switch (vectors) {
+    case 8: read_sum_packed_kernel<T, 8><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    case 16: read_sum_packed_kernel<T, 16><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    case 32: read_sum_packed_kernel<T, 32><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    case 64: read_sum_packed_kernel<T, 64><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    case 128: read_sum_packed_kernel<T, 128><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    case 256: read_sum_packed_kernel<T, 256><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
+    default: read_sum_kernel<T, kVec><<<g, b, 0, stream>>>(s, sink, elements, block_elements, segments, serial);
   }
   return launch_status("read_sum_kernel");
 }
