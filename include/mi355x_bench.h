@@ -109,8 +109,9 @@ int mb_clock_witness(uint64_t* out, uint64_t out_bytes, uint32_t microseconds, v
  * `block_threads` is a multiple of 64 up to 1024; each workgroup moves
  * `block_threads * vectors_per_thread * 16` bytes per step. `grid_blocks` = 0
  * launches one workgroup per step (the reference's grid = cdiv(N, BLOCK));
- * otherwise that many workgroups stride over the buffer. A tail shorter than
- * 16 bytes, or pointers without 16-byte alignment, take narrower accesses.
+ * otherwise that many workgroups stride over the buffer. The bytes before an
+ * unaligned dst's first whole 128-byte line and a tail shorter than 16 bytes
+ * are moved one by one in the same launch.
  * Replaces: bench_bandwidth.py:36-47 (copy_kernel, launch_copy). */
 int mb_copy(const void* src, void* dst, uint64_t bytes, uint32_t block_threads,
             uint32_t vectors_per_thread, uint32_t grid_blocks, uint32_t flags, void* stream);

@@ -33,6 +33,7 @@ _GEMM_RING_RE = re.compile(r"gemm_ring_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)EL
 _GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)E(?:Lb([01])E)?E")
 _ELEM_BITS = {"bf16": 16, "f16": 16, "i8": 8, "fp8": 8, "mxfp4": 4, "f32": 32, "f64": 64}
 _COPY_RE = re.compile(r"copy_kernelI(Dv4_j|j|h)Li(\d+)ELi([012])E")
+_COPY_EDGES_RE = re.compile(r"copy_edges_kernelILi(\d+)ELi([012])E")
 _READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)Li(\d+)E")
 _READ_PACKED_RE = re.compile(r"read_sum_packed_kernelI(f|DF16_|t)Li(\d+)E")
 _VECTOR_RE = re.compile(r"vector_(\w+?)_kernelILi(\d+)E")
@@ -72,6 +73,10 @@ def registered_name(symbol: str) -> str | None:
     if match:
         unit, vpt, policy = match.groups()
         return f"copy_{_COPY_UNIT[unit]}_vpt{vpt}{('', '_nt', '_stream')[int(policy)]}"
+    match = _COPY_EDGES_RE.search(symbol)
+    if match:
+        vpt, policy = match.groups()
+        return f"copy_edges_vpt{vpt}{('', '_nt', '_stream')[int(policy)]}"
     match = _READ_PACKED_RE.search(symbol)
     if match:
         dtype, vectors = match.groups()

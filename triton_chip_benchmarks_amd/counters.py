@@ -139,6 +139,8 @@ def registered_name(demangled: str) -> str:
         unit = "dwordx4" if "__vector(4)" in args[0] else "byte" if "char" in args[0] else "dword"
         policy = {"0": "", "false": "", "1": "_nt", "true": "_nt", "2": "_stream"}[args[2]]
         return f"copy_{unit}_vpt{args[1]}{policy}"
+    if family == "copy_edges_kernel":
+        return f"copy_edges_vpt{args[0]}{('', '_nt', '_stream')[int(args[1])]}"
     if family in ("read_sum_kernel", "read_sum_packed_kernel"):
         kind = {"float": "f32", "_Float16": "f16", "__bf16": "bf16", "unsigned short": "bf16"}.get(args[0], args[0])
         return f"read_sum_{kind}_{'vec' if family == 'read_sum_kernel' else 'packed' + args[1]}"

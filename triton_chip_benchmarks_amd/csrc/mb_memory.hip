@@ -1,6 +1,6 @@
 // HBM copy and read kernels (memory_bandwidth row).
 //
-// Copy: every lane moves 16-byte vectors (global_load_dwordx4 /
+// Copy: every lane moves 16-byte vectors, at any address (global_load_dwordx4 /
 // global_store_dwordx4); consecutive lanes touch consecutive vectors, so each
 // wave64 instruction covers 1 KiB of contiguous memory. A workgroup step holds
 // `vectors_per_thread` independent loads in flight before the stores. The
@@ -27,25 +27,31 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Copy cache policies.
 constexpr int kPlain = 0, kNontemporal = 1, kStream = 2;
 
-template <typename T, int POLICY>
-__device__ __forceinline__ T load_elem(const T* ptr) {
-  if constexpr (POLICY != kPlain) return __builtin_nontemporal_load(ptr);
-  return *ptr;
+// 16 bytes at any address: gfx950 takes a global_load_dwordx4 there.
+typedef u32x4 u32x4_unaligned __attribute__((aligned(1)));
+
+template <int POLICY, bool UNALIGNED>
+__device__ __forceinline__ u32x4 load_elem(const u32x4* ptr) {
+  if constexpr (UNALIGNED) {
+    const u32x4_unaligned* at = reinterpret_cast<const u32x4_unaligned*>(ptr);
+    if constexpr (POLICY != kPlain) return __builtin_nontemporal_load(at);
+    return *at;
+  } else {
+    if constexpr (POLICY != kPlain) return __builtin_nontemporal_load(ptr);
+    return *ptr;
+  }
 }
 
-// Device-scope (sc1) vector stores; the compiler has no builtin for the scope bits.
+// Device-scope (sc1) vector stores; the compiler has no builtin for the scope
+// bits. A store of more than 8 bytes needs one wait state before a VALU
+// instruction rewrites its data registers, which the compiler cannot see to
+// behind inline assembly.
 __device__ __forceinline__ void store_sc1(u32x4* ptr, u32x4 value) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(ptr), "v"(value) : "memory");
-}
-__device__ __forceinline__ void store_sc1(uint32_t* ptr, uint32_t value) {
-  asm volatile("global_store_dword %0, %1, off sc1" ::"v"(ptr), "v"(value) : "memory");
-}
-__device__ __forceinline__ void store_sc1(uint8_t* ptr, uint8_t value) {
-  asm volatile("global_store_byte %0, %1, off sc1" ::"v"(ptr), "v"(static_cast<uint32_t>(value)) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(ptr), "v"(value) : "memory");
 }
 
-template <typename T, int POLICY>
-__device__ __forceinline__ void store_elem(T* ptr, T value) {
+template <int POLICY>
+__device__ __forceinline__ void store_elem(u32x4* ptr, u32x4 value) {
   if constexpr (POLICY == kStream) {
     store_sc1(ptr, value);
   } else if constexpr (POLICY == kNontemporal) {
@@ -55,11 +61,12 @@ __device__ __forceinline__ void store_elem(T* ptr, T value) {
   }
 }
 
-// T is the access unit (u32x4, uint32_t or uint8_t); n counts units.
-template <typename T, int VPT, int POLICY>
-__global__ void __launch_bounds__(1024) copy_kernel(const T* __restrict__ src, T* __restrict__ dst,
-                                                     uint64_t n) {
-  const uint32_t block_threads = blockDim.x;
+// n 16-byte vectors; dst is 16-byte aligned, src unless UNALIGNED too. The
+// kernels pass blockDim.x: read in here, it costs every wave a load (the
+// compiler then allows for a partial last workgroup; 1 GiB 330 us, not 316).
+template <int VPT, int POLICY, bool UNALIGNED>
+__device__ __forceinline__ void copy_vectors(const u32x4* __restrict__ src, u32x4* __restrict__ dst, uint64_t n,
+                                             uint32_t block_threads) {
   const uint64_t step = static_cast<uint64_t>(block_threads) * VPT;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * step;
   for (uint64_t base = blockIdx.x * step + threadIdx.x; base < n; base += stride) {
@@ -68,27 +75,53 @@ __global__ void __launch_bounds__(1024) copy_kernel(const T* __restrict__ src, T
     // SGPR file at 16 vectors per lane and spills.
     uint32_t threads = block_threads;
     asm("" : "+s"(threads));
-    const T* s = src + base;
-    T* d = dst + base;
+    const u32x4* s = src + base;
+    u32x4* d = dst + base;
     const uint64_t left = n - base;
-    T values[VPT];
+    u32x4 values[VPT];
     if (left > static_cast<uint64_t>(VPT - 1) * threads) {
 #pragma unroll
-      for (int j = 0; j < VPT; ++j) values[j] = load_elem<T, POLICY>(s + j * threads);
+      for (int j = 0; j < VPT; ++j) values[j] = load_elem<POLICY, UNALIGNED>(s + j * threads);
 #pragma unroll
-      for (int j = 0; j < VPT; ++j) store_elem<T, POLICY>(d + j * threads, values[j]);
+      for (int j = 0; j < VPT; ++j) store_elem<POLICY>(d + j * threads, values[j]);
     } else {
 #pragma unroll
       for (int j = 0; j < VPT; ++j)
-        if (j * threads < left) values[j] = load_elem<T, POLICY>(s + j * threads);
+        if (j * threads < left) values[j] = load_elem<POLICY, UNALIGNED>(s + j * threads);
 #pragma unroll
       for (int j = 0; j < VPT; ++j)
-        if (j * threads < left) store_elem<T, POLICY>(d + j * threads, values[j]);
+        if (j * threads < left) store_elem<POLICY>(d + j * threads, values[j]);
     }
   }
 }
 
-// Bytes after the last whole 16-byte vector.
+// T is the access unit (u32x4); n counts units.
+template <typename T, int VPT, int POLICY>
+__global__ void __launch_bounds__(1024) copy_kernel(const T* __restrict__ src, T* __restrict__ dst,
+                                                     uint64_t n) {
+  copy_vectors<VPT, POLICY, false>(src, dst, n, blockDim.x);
+}
+
+// A copy with `head` bytes before and `tail` bytes after its n whole vectors,
+// which the first workgroup moves: dst + head is 16-byte aligned, src + head
+// need not be. One launch where the body and its tail took two (8 MiB and a
+// tail 6.5 -> 5.2 us), and 16-byte accesses where unaligned pointers took single
+// dwords or bytes (1 GiB, one wave a workgroup, streaming: on dwords 888 -> 330
+// us, on bytes 3531 -> 331; aligned it takes 317).
+template <int VPT, int POLICY>
+__global__ void __launch_bounds__(1024)
+    copy_edges_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint64_t n, uint32_t head,
+                      uint32_t tail) {
+  copy_vectors<VPT, POLICY, true>(reinterpret_cast<const u32x4*>(src + head), reinterpret_cast<u32x4*>(dst + head), n,
+                                  blockDim.x);
+  if (blockIdx.x == 0) {
+    const uint64_t after = head + n * 16;
+    for (uint32_t i = threadIdx.x; i < head; i += blockDim.x) dst[i] = src[i];
+    if (threadIdx.x < tail) dst[after + threadIdx.x] = src[after + threadIdx.x];
+  }
+}
+
+// A copy of less than one whole vector.
 __global__ void copy_tail_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t n) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
@@ -96,16 +129,20 @@ __global__ void copy_tail_kernel(const uint8_t* __restrict__ src, uint8_t* __res
 // Write-only stream (the copy's store half): every 32-bit word of dst becomes
 // `pattern`, one 16-byte store per lane per trip, grid-stride, with the copy's
 // store policies.
+// The `tail` bytes after them are the first workgroup's; byte i of the buffer
+// is byte (i % 4) of the little-endian pattern (the tail starts 16-aligned).
 template <int POLICY>
-__global__ void __launch_bounds__(1024) fill_kernel(u32x4* __restrict__ dst, uint64_t n, uint32_t pattern) {
+__global__ void __launch_bounds__(1024)
+    fill_kernel(u32x4* __restrict__ dst, uint64_t n, uint32_t pattern, uint32_t tail) {
   const u32x4 value = {pattern, pattern, pattern, pattern};
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n; i += stride)
-    store_elem<u32x4, POLICY>(dst + i, value);
+    store_elem<POLICY>(dst + i, value);
+  if (blockIdx.x == 0 && threadIdx.x < tail)
+    reinterpret_cast<uint8_t*>(dst + n)[threadIdx.x] = static_cast<uint8_t>(pattern >> (8 * (threadIdx.x & 3)));
 }
 
-// Bytes after the last whole 16-byte vector of a fill; byte i of the buffer
-// is byte (i % 4) of the little-endian pattern (the tail starts 16-aligned).
+// A fill of less than one whole vector.
 __global__ void fill_tail_kernel(uint8_t* __restrict__ dst, uint32_t n, uint32_t pattern) {
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = static_cast<uint8_t>(pattern >> (8 * (i & 3)));
 }
@@ -139,9 +176,6 @@ __device__ __forceinline__ float wave_sum(float value) {
   for (int offset = 32; offset > 0; offset >>= 1) value += __shfl_xor(value, offset, 64);
   return value;
 }
-
-// 16 bytes at any address: gfx950 takes a global_load_dwordx4 there.
-typedef u32x4 u32x4_unaligned __attribute__((aligned(1)));
 
 template <typename T>
 __device__ __forceinline__ u32x4 load_vector(const T* ptr) {
@@ -312,44 +346,55 @@ __global__ void __launch_bounds__(1024) read_sum_kernel(const T* __restrict__ sr
   }
 }
 
-template <typename T, int POLICY>
-int launch_copy_units(const void* src, void* dst, uint64_t units, uint32_t threads, uint32_t vpt,
-                      uint32_t grid_blocks, hipStream_t stream) {
+// Launches the aligned kernel (head = tail = 0 and src aligned) or the one with
+// edges over `vectors` whole vectors.
+template <int VPT, int POLICY>
+void launch_copy_kernel(const char* src, char* dst, uint64_t vectors, uint32_t head, uint32_t tail, dim3 grid,
+                        dim3 threads, hipStream_t stream) {
+  if (head == 0 && tail == 0 && aligned(src, 16))
+    copy_kernel<u32x4, VPT, POLICY><<<grid, threads, 0, stream>>>(reinterpret_cast<const u32x4*>(src),
+                                                                  reinterpret_cast<u32x4*>(dst), vectors);
+  else
+    copy_edges_kernel<VPT, POLICY><<<grid, threads, 0, stream>>>(reinterpret_cast<const uint8_t*>(src),
+                                                                 reinterpret_cast<uint8_t*>(dst), vectors, head, tail);
+}
+
+template <int POLICY>
+int launch_copy(const char* src, char* dst, uint64_t vectors, uint32_t head, uint32_t tail, uint32_t threads,
+                uint32_t vpt, uint32_t grid_blocks, hipStream_t stream) {
   const uint64_t step = static_cast<uint64_t>(threads) * vpt;
-  const uint64_t steps = (units + step - 1) / step;
-  uint64_t grid = grid_blocks ? (grid_blocks < steps ? grid_blocks : steps) : steps;
-  if (grid == 0) return MB_OK;
+  const uint64_t steps = (vectors + step - 1) / step;
+  const uint64_t grid = grid_blocks ? (grid_blocks < steps ? grid_blocks : steps) : steps;
   if (grid > 0x7fffffffull)
     return fail(MB_ERR_INVALID, "mb_copy: %llu workgroups exceed the grid limit; raise vectors_per_thread",
                 static_cast<unsigned long long>(grid));
-  const T* s = static_cast<const T*>(src);
-  T* d = static_cast<T*>(dst);
   dim3 g(static_cast<uint32_t>(grid)), b(threads);
   switch (vpt) {
-    case 1: copy_kernel<T, 1, POLICY><<<g, b, 0, stream>>>(s, d, units); break;
-    case 2: copy_kernel<T, 2, POLICY><<<g, b, 0, stream>>>(s, d, units); break;
-    case 4: copy_kernel<T, 4, POLICY><<<g, b, 0, stream>>>(s, d, units); break;
-    case 8: copy_kernel<T, 8, POLICY><<<g, b, 0, stream>>>(s, d, units); break;
-    case 16: copy_kernel<T, 16, POLICY><<<g, b, 0, stream>>>(s, d, units); break;
+    case 1: launch_copy_kernel<1, POLICY>(src, dst, vectors, head, tail, g, b, stream); break;
+    case 2: launch_copy_kernel<2, POLICY>(src, dst, vectors, head, tail, g, b, stream); break;
+    case 4: launch_copy_kernel<4, POLICY>(src, dst, vectors, head, tail, g, b, stream); break;
+    case 8: launch_copy_kernel<8, POLICY>(src, dst, vectors, head, tail, g, b, stream); break;
+    case 16: launch_copy_kernel<16, POLICY>(src, dst, vectors, head, tail, g, b, stream); break;
     default: return fail(MB_ERR_INVALID, "mb_copy: vectors_per_thread %u not in {1,2,4,8,16}", vpt);
   }
   return launch_status("copy_kernel");
 }
 
-#define MB_REGISTER_COPY_POLICY(T, TNAME, P, SUFFIX)                                          \
-  MB_REGISTER_KERNEL("copy_" TNAME "_vpt1" SUFFIX, (copy_kernel<T, 1, P>));                  \
-  MB_REGISTER_KERNEL("copy_" TNAME "_vpt2" SUFFIX, (copy_kernel<T, 2, P>));                  \
-  MB_REGISTER_KERNEL("copy_" TNAME "_vpt4" SUFFIX, (copy_kernel<T, 4, P>));                  \
-  MB_REGISTER_KERNEL("copy_" TNAME "_vpt8" SUFFIX, (copy_kernel<T, 8, P>));                  \
-  MB_REGISTER_KERNEL("copy_" TNAME "_vpt16" SUFFIX, (copy_kernel<T, 16, P>))
-#define MB_REGISTER_COPY(T, TNAME)                                                            \
-  MB_REGISTER_COPY_POLICY(T, TNAME, kPlain, "");                                              \
-  MB_REGISTER_COPY_POLICY(T, TNAME, kNontemporal, "_nt");                                     \
-  MB_REGISTER_COPY_POLICY(T, TNAME, kStream, "_stream")
+#define MB_REGISTER_COPY(P, SUFFIX)                                                         \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt1" SUFFIX, (copy_kernel<u32x4, 1, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt2" SUFFIX, (copy_kernel<u32x4, 2, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt4" SUFFIX, (copy_kernel<u32x4, 4, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt8" SUFFIX, (copy_kernel<u32x4, 8, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt16" SUFFIX, (copy_kernel<u32x4, 16, P>));             \
+  MB_REGISTER_KERNEL("copy_edges_vpt1" SUFFIX, (copy_edges_kernel<1, P>));                  \
+  MB_REGISTER_KERNEL("copy_edges_vpt2" SUFFIX, (copy_edges_kernel<2, P>));                  \
+  MB_REGISTER_KERNEL("copy_edges_vpt4" SUFFIX, (copy_edges_kernel<4, P>));                  \
+  MB_REGISTER_KERNEL("copy_edges_vpt8" SUFFIX, (copy_edges_kernel<8, P>));                  \
+  MB_REGISTER_KERNEL("copy_edges_vpt16" SUFFIX, (copy_edges_kernel<16, P>))
 
-MB_REGISTER_COPY(u32x4, "dwordx4");
-MB_REGISTER_COPY(uint32_t, "dword");
-MB_REGISTER_COPY(uint8_t, "byte");
+MB_REGISTER_COPY(kPlain, "");
+MB_REGISTER_COPY(kNontemporal, "_nt");
+MB_REGISTER_COPY(kStream, "_stream");
 MB_REGISTER_KERNEL("copy_tail", copy_tail_kernel);
 MB_REGISTER_KERNEL("fill_dwordx4", (fill_kernel<kPlain>));
 MB_REGISTER_KERNEL("fill_dwordx4_nt", (fill_kernel<kNontemporal>));
@@ -424,30 +469,23 @@ int mb_copy(const void* src, void* dst, uint64_t bytes, uint32_t block_threads, 
   // makes both loads and stores non-temporal.
   const int policy = (flags & MB_COPY_WRITE_THROUGH) ? kStream : (flags & MB_COPY_NONTEMPORAL) ? kNontemporal : kPlain;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  auto units = [&](auto unit, const void* from, void* to, uint64_t count) {
-    using T = decltype(unit);
-    switch (policy) {
-      case kStream: return launch_copy_units<T, kStream>(from, to, count, block_threads, vectors_per_thread,
-                                                         grid_blocks, st);
-      case kNontemporal: return launch_copy_units<T, kNontemporal>(from, to, count, block_threads,
-                                                                   vectors_per_thread, grid_blocks, st);
-      default: return launch_copy_units<T, kPlain>(from, to, count, block_threads, vectors_per_thread,
-                                                   grid_blocks, st);
-    }
-  };
-  if (aligned(src, 16) && aligned(dst, 16)) {
-    const uint64_t vectors = bytes / 16;
-    if (int rc = units(u32x4{}, src, dst, vectors)) return rc;
-    const uint32_t tail = static_cast<uint32_t>(bytes % 16);
-    if (tail) {
-      copy_tail_kernel<<<1, 64, 0, st>>>(reinterpret_cast<const uint8_t*>(s + vectors * 16),
-                                         reinterpret_cast<uint8_t*>(d + vectors * 16), tail);
-      return launch_status("copy_tail_kernel");
-    }
-    return MB_OK;
+  // The head brings unaligned stores to whole 128-byte lines; an aligned dst
+  // keeps its vectors where they are.
+  const uint32_t head = aligned(dst, 16) ? 0 : static_cast<uint32_t>(-reinterpret_cast<uintptr_t>(dst) & 127);
+  const uint64_t vectors = bytes > head ? (bytes - head) / 16 : 0;
+  if (vectors == 0) {
+    copy_tail_kernel<<<1, 64, 0, st>>>(reinterpret_cast<const uint8_t*>(s), reinterpret_cast<uint8_t*>(d),
+                                       static_cast<uint32_t>(bytes));
+    return launch_status("copy_tail_kernel");
   }
-  if (aligned(src, 4) && aligned(dst, 4) && bytes % 4 == 0) return units(uint32_t{}, src, dst, bytes / 4);
-  return units(uint8_t{}, src, dst, bytes);
+  const uint32_t tail = static_cast<uint32_t>((bytes - head) % 16);
+  switch (policy) {
+    case kStream: return launch_copy<kStream>(s, d, vectors, head, tail, block_threads, vectors_per_thread,
+                                              grid_blocks, st);
+    case kNontemporal: return launch_copy<kNontemporal>(s, d, vectors, head, tail, block_threads, vectors_per_thread,
+                                                        grid_blocks, st);
+    default: return launch_copy<kPlain>(s, d, vectors, head, tail, block_threads, vectors_per_thread, grid_blocks, st);
+  }
 }
 
 int mb_fill(void* dst, uint64_t bytes, uint32_t pattern, uint32_t block_threads, uint32_t grid_blocks,
@@ -468,19 +506,16 @@ int mb_fill(void* dst, uint64_t bytes, uint32_t pattern, uint32_t block_threads,
     return fail(MB_ERR_INVALID, "mb_fill: %llu workgroups exceed the grid limit; pass grid_blocks",
                 static_cast<unsigned long long>(grid));
   u32x4* d = static_cast<u32x4*>(dst);
-  if (grid) {
-    dim3 g(static_cast<uint32_t>(grid)), b(block_threads);
-    if (flags & MB_COPY_WRITE_THROUGH) fill_kernel<kStream><<<g, b, 0, st>>>(d, vectors, pattern);
-    else if (flags & MB_COPY_NONTEMPORAL) fill_kernel<kNontemporal><<<g, b, 0, st>>>(d, vectors, pattern);
-    else fill_kernel<kPlain><<<g, b, 0, st>>>(d, vectors, pattern);
-    if (int rc = launch_status("fill_kernel")) return rc;
-  }
   const uint32_t tail = static_cast<uint32_t>(bytes % 16);
-  if (tail) {
-    fill_tail_kernel<<<1, 64, 0, st>>>(static_cast<uint8_t*>(dst) + vectors * 16, tail, pattern);
+  if (grid == 0) {
+    fill_tail_kernel<<<1, 64, 0, st>>>(static_cast<uint8_t*>(dst), tail, pattern);
     return launch_status("fill_tail_kernel");
   }
-  return MB_OK;
+  dim3 g(static_cast<uint32_t>(grid)), b(block_threads);
+  if (flags & MB_COPY_WRITE_THROUGH) fill_kernel<kStream><<<g, b, 0, st>>>(d, vectors, pattern, tail);
+  else if (flags & MB_COPY_NONTEMPORAL) fill_kernel<kNontemporal><<<g, b, 0, st>>>(d, vectors, pattern, tail);
+  else fill_kernel<kPlain><<<g, b, 0, st>>>(d, vectors, pattern, tail);
+  return launch_status("fill_kernel");
 }
 
 int mb_read_sum(int dtype, const void* src, float* sink, uint64_t elements, uint32_t block_elements,
