@@ -289,9 +289,12 @@ def gemm(dtype: str, config: dict, a, b, c, m: int, n: int, k: int, scale_a=None
 
 
 def stream_handle(stream=None) -> int | None:
-    """The raw hipStream_t of a torch stream (the current one by default)."""
+    """The raw hipStream_t of a torch stream (the current one of the current device by default)."""
     import torch
 
+    if stream is None and torch.cuda.is_initialized():
+        # Without building a torch.cuda.Stream object, which takes 2.8 us of a 7.4 us copy call; this takes 0.4.
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()) or None
     if stream is None:
         stream = torch.cuda.current_stream()
     handle = stream.cuda_stream
