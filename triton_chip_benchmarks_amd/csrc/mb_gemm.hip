@@ -489,10 +489,10 @@ __global__ void __launch_bounds__(256)
 // program order is the issue order.
 //
 // RAGGED takes any shape, as the ring kernels do: DMAs and stores past M, N or
-// K get out-of-range offsets from the buffer bounds check, and an odd step
-// count is rounded up with a step of zeros. Its row offsets sit in registers
-// instead of the scalar offset, which the bounds check subtracts from the
-// buffer's size and must not exceed it.
+// K get out-of-range offsets from the buffer bounds check, and the last of an
+// odd number of steps runs by itself. Its row offsets sit in registers instead
+// of the scalar offset, which the bounds check subtracts from the buffer's size
+// and must not exceed it.
 template <class Op, bool RAGGED>
 __global__ void __launch_bounds__(256)
     gemm_dma_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, const uint8_t* __restrict__,
@@ -644,10 +644,12 @@ __global__ void __launch_bounds__(256)
     });
     slot = next_slot;
   };
-  for (int kt = 0; kt < k_steps; kt += 2) {
+  int kt = 0;
+  for (; kt + 1 < k_steps; kt += 2) {
     step(kt, 0);
     step(kt + 1, 1);
   }
+  if (RAGGED && kt < k_steps) step(kt, 0);
 #pragma unroll
   for (int i = 0; i < TILES; ++i)
 #pragma unroll
@@ -658,19 +660,20 @@ __global__ void __launch_bounds__(256)
     constexpr int ES = sizeof(typename Op::Out);
     const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
         C + static_cast<int64_t>(m0) * N + n0, (short)0, min(BM, M - m0) * N * ES - n0 * ES, kBufferWord3);
+    // A row's eight 64-byte pieces one after the other: rows off the 128-byte
+    // grid share lines between pieces (FP8 8191x8191x8192 431 -> 378 us).
 #pragma unroll
-    for (int j = 0; j < TILES; ++j) {
-      const int col = wn * 128 + j * Op::N + lrow;
-      const bool inside = n0 + col < N;
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-      for (int i = 0; i < TILES; ++i)
+      for (int r = 0; r < Op::ACC_REGS; ++r)
 #pragma unroll
-        for (int r = 0; r < Op::ACC_REGS; ++r) {
+        for (int j = 0; j < TILES; ++j) {
+          const int col = wn * 128 + j * Op::N + lrow;
           const int offset = ((wm * 128 + i * Op::M + Op::out_row(lane, r)) * N + col) * ES;
           const typename Op::Out value = acc[i][j][r];
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rc, inside ? offset : kOutOfRange, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rc, n0 + col < N ? offset : kOutOfRange,
+                                                0, 0);
         }
-    }
   } else {
 #pragma unroll
   for (int i = 0; i < TILES; ++i)

@@ -9,10 +9,15 @@ namespace mb {
 // Cache policy of the C stores: written through the XCD's L2 (device scope,
 // sc1). The tiles of a round end together, and lines left dirty would wait in
 // the L2 for the flush at the kernel's end. 2048^3 (us): BF16 20.96 -> 19.77,
-// MXFP4 10.43 -> 9.24; 1024^3 BF16 5.51 -> 5.13. Each store instruction writes
-// whole 128-byte lines here; the 256x256 kernels' 64-byte rows lose by it (FP8
-// 5000x3000x4112 61.5 -> 68.3). Non-temporal stores gain as much at 2048^3, but
-// MXFP4 4096^3 on 256x128 tiles takes 50.4 with them, 45.8 with sc1, 47.9 plain.
+// MXFP4 10.43 -> 9.24; 1024^3 BF16 5.51 -> 5.13. Where an output of many rounds
+// has rows of partial 128-byte lines, which stores then share, plain stores are
+// better (BF16 7000x9001x1040 179, with sc1 236), as they are for the 256x256
+// kernels' 64-byte stores (FP8 5000x3000x4112 61.5, with sc1 68.3).
+// Non-temporal stores gain as much at 2048^3, but MXFP4 4096^3 on 256x128 tiles
+// takes 50.4 with them, 45.8 with sc1, 47.9 plain.
+// Order: such outputs store a row's pieces one after the other, so that shared
+// lines are completed at once (the 179, column blocks outermost: 197); in few
+// rounds, column blocks outermost is better (2048^3 BF16 20.0, rows 21.5).
 constexpr int kStoreThrough = 16;
 
 template <class Op, int BM, int BN, int STAGES>
@@ -28,6 +33,8 @@ struct RingTile {
   static constexpr int OPERANDS = (BM + BN) * ROWB;
   static constexpr int SCALES_A = BM > 128 ? 2048 : 1024;  // bytes: 8 per row, in whole DMAs
   static constexpr int STAGE = OPERANDS + (Op::SCALED ? SCALES_A + 1024 : 0);
+  // The tiles that large outputs run on; the others are launched for few rounds.
+  static constexpr bool MANY_ROUNDS = BM > 128 || STAGES == 2;
   static constexpr int MFMAS = FM * FN * PER, READS = (FM + FN) * CHUNKS;
   static_assert(Op::M == Op::N && WM % Op::M == 0 && WN % Op::N == 0, "whole instructions per wave");
   static_assert(BM % 64 == 0 && BN % 64 == 0 && BM <= 256 && BN <= 128, "whole DMAs per wave; scale rows per stage");
@@ -264,22 +271,36 @@ __global__ void __launch_bounds__(256)
   constexpr int ES = sizeof(typename Op::Out);
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
       C + static_cast<int64_t>(m0) * N + n0, (short)0, min(BM, M - m0) * N * ES - n0 * ES, kBufferWord3);
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
+  auto store = [&](int i, int j, int r, auto policy_c) __attribute__((always_inline)) {
+    constexpr int policy = decltype(policy_c)::value;
     const int col = wn * T::WN + j * Op::N + lane % Op::N;
-    const bool inside = n0 + col < N;
+    const int offset = ((wm * T::WM + i * Op::M + Op::out_row(lane, r)) * N + col) * ES;
+    const int at = n0 + col < N ? offset : kOutOfRange;
+    const typename Op::Out value = acc[i][j][r];
+    if constexpr (ES == 8)
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, value), rc, at, 0, policy);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rc, at, 0, policy);
+  };
+  auto store_rows = [&](auto policy_c) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int r = 0; r < Op::ACC_REGS; ++r) {
-        const int offset = ((wm * T::WM + i * Op::M + Op::out_row(lane, r)) * N + col) * ES;
-        const int at = inside ? offset : kOutOfRange;
-        const typename Op::Out value = acc[i][j][r];
-        if constexpr (ES == 8)
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, value), rc, at, 0, kStoreThrough);
-        else
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, value), rc, at, 0, kStoreThrough);
-      }
+      for (int r = 0; r < Op::ACC_REGS; ++r)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) store(i, j, r, policy_c);
+  };
+  if constexpr (!T::MANY_ROUNDS) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int r = 0; r < Op::ACC_REGS; ++r) store(i, j, r, std::integral_constant<int, kStoreThrough>{});
+  } else if ((static_cast<int64_t>(N) * ES | reinterpret_cast<intptr_t>(C)) % 128 == 0) {
+    store_rows(std::integral_constant<int, kStoreThrough>{});
+  } else {
+    store_rows(std::integral_constant<int, 0>{});
   }
 #endif
 }
