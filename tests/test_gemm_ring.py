@@ -157,3 +157,46 @@ def test_mxfp4_scales_off_the_16_byte_grid(gpu, offset, checked):
     _native.gemm("fp4", config, *(torch.from_numpy(ot.pack_e2m1(x)).cuda() for x in codes), c, m, n, k, *scales)
     torch.cuda.synchronize()
     assert np.array_equal(c.cpu().numpy().astype(np.float64), ot.gemm_reference(values[0], values[1].T))
+
+
+def _ring_kernels():
+    """(name, stages, DMAs per wave and step) of every ring kernel."""
+    from triton_chip_benchmarks_amd import _native, audit
+
+    out = []
+    for name in _native.kernel_names():
+        symbol = audit.symbols().get(name, "")
+        match = audit._GEMM_RING_RE.search(symbol)
+        if match:
+            _, bm, bn, stages = match.groups()
+            out.append((name, int(stages), int(bm) // 32 + int(bn) // 32 + ("mxfp4" in name)))
+    return out
+
+
+def test_ring_loops_wait_for_every_dma_and_every_read():
+    """In the compiled loops, an LDS-DMA is retired by the waits within STAGES-1 barriers of its issue, after which
+    its stage is read (one barrier less would be too few where the ring has a third stage), and every barrier,
+    after which a stage just read is refilled, follows a wait for all LDS reads."""
+    from test_audit import _dma_coverage_violations
+    from triton_chip_benchmarks_amd import audit
+
+    kernels = _ring_kernels()
+    assert len(kernels) == 25
+    for name, stages, dmas in kernels:
+        body = audit.hot_loop(name)
+        assert sum(line.rstrip().endswith(" lds") for line in body) == 2 * dmas, name
+        assert sum(audit.mnemonic(line) == "s_barrier" for line in body) == 2, name
+        assert _dma_coverage_violations(body, horizon=stages - 1) == [], name
+        if stages > 2:
+            assert _dma_coverage_violations(body, horizon=stages - 2), name
+        unwaited = [line for line in body if not (audit.mnemonic(line) == "s_waitcnt" and "vmcnt" in line)]
+        assert _dma_coverage_violations(unwaited, horizon=stages - 1), name
+        # The reads of a step are all waited for before its closing barrier.
+        pending = False
+        for line in body + body:
+            if audit.mnemonic(line).startswith("ds_read"):
+                pending = True
+            elif audit.mnemonic(line) == "s_waitcnt" and "lgkmcnt(0)" in line:
+                pending = False
+            elif audit.mnemonic(line) == "s_barrier":
+                assert not pending, name

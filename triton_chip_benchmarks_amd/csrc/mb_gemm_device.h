@@ -63,8 +63,15 @@ __device__ __forceinline__ void band_tile_any(int tiles_m, int tiles_n, int grou
 // maxima, which wait for nothing.
 constexpr int vmcnt_only(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-// Barrier that orders LDS only: global loads in flight stay in flight across it.
+// s_waitcnt's immediate for lgkmcnt(0) alone.
+constexpr int kLgkmcntZero = 15 | (3 << 14) | (7 << 4);
+
+// Barrier that orders LDS only: global loads in flight stay in flight across
+// it. The LDS reads before it are waited for explicitly: at a loop's head the
+// compiler drops the wait that the release fence asks for when nothing is
+// outstanding on the way into the loop, though reads of the last trip are.
 __device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(kLgkmcntZero);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
