@@ -63,12 +63,16 @@ struct RingTile {
 // kt+1 and the DMAs of step kt+STAGES into stage kt % STAGES. A stage is thus
 // refilled STAGES-1 steps before it is needed.
 //
-// What bounds it: below the LDS, the matrix cores for FP32 and FP64 (a step's
-// MFMAs take 4096 cycles at 128x128). For the narrower formats they take 512,
-// in which the LDS serves 64 KiB of fragment reads (512 cycles) and takes
-// 32 KiB from the DMAs: a full chip measures 0.43-0.48 us (about 1030 cycles)
-// a step. 256x128 moves 25% less per output; 64x64 moves twice as much, but
-// fills the chip from 1024^3 on. Stages: 128x128 needs 4 for its latency when
+// What bounds it: the matrix cores for FP32 and FP64 (a step's MFMAs take 4096
+// cycles at 128x128; FP64 2048^3 runs at 89% of their rate, a few hundred cycles
+// a step go to its barrier). For the narrower formats they take 512, and a full
+// chip measures 0.43-0.48 us (about 1030 cycles) a step: 32 KiB per CU, 19 TB/s
+// from the L2s, of which 5 TB/s cross the fabric at 2048^3 (67 MB: each XCD
+// fetches its own copy of its panels). Splitting a step's K over the waves, which
+// halves the LDS reads (64 KiB, 512 cycles), takes 4% off a step and adds a
+// final sum: 18.9 -> 19.8 us at 2048^3. 256x128 moves 25% less per output;
+// 64x64 moves twice as much, but fills the chip from 1024^3 on. Stages: 128x128
+// needs 4 for its latency when
 // a CU holds one tile (2048^3 BF16: 25.6 us with 2, 24 with 3, 20.9 with 4, 23
 // with 5) and 2 when it can hold a pair, whose prologues and stores overlap
 // (4096^3: 118 us with 2, 129 with 4); 64x64 gains nothing from more than 3
