@@ -213,8 +213,9 @@ const char* mb_gemm_kernel_name(int format, const mb_gemm_config* config);
  * past K are ignored): one 256-element K step of a tile reads one contiguous
  * run of 8 bytes per row. K * element bits must be a multiple of 128 (16-byte
  * rows). group_m = 0 selects the launched kernel's default band height (tile
- * rows per band: 8, or the measured best of its exact-shape kernel: 4 for BF16
- * and FP16, 6 for FP8 and 7 for INT8 256x256);
+ * rows per band: 8, or the kernel's measured best: 6 for 128x128, 4 for 256x128
+ * and for the exact-shape 256x256 of BF16 and FP16, 6 for that of FP8, 7 for
+ * that of INT8);
  * a band taller than the tile rows acts as the full height. The band height
  * orders the tiles only: every value gives the same C.
  * Replaces: bench_tensor.py:172-209 (_gemm_kernel) and 235-246 (_launch),
