@@ -67,8 +67,8 @@ struct RingTile {
 // cycles at 128x128; FP64 2048^3 runs at 89% of their rate, a few hundred cycles
 // a step go to its barrier). For the narrower formats they take 512, and a full
 // chip measures 0.43-0.48 us (about 1030 cycles) a step: 32 KiB per CU, 19 TB/s
-// from the L2s, of which 5 TB/s cross the fabric at 2048^3 (67 MB: each XCD
-// fetches its own copy of its panels). Splitting a step's K over the waves, which
+// from the L2s, of which about 4 TB/s cross the fabric at 2048^3 (50 MB of reads:
+// each XCD fetches its own copy of its 12 panels). Splitting a step's K over the waves, which
 // halves the LDS reads (64 KiB, 512 cycles), takes 4% off a step and adds a
 // final sum: 18.9 -> 19.8 us at 2048^3. 256x128 moves 25% less per output;
 // 64x64 moves twice as much, but fills the chip from 1024^3 on. Stages: 128x128

@@ -13,13 +13,15 @@ void launch_ring(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const ui
       a, b, sa, sb, static_cast<typename Op::Out*>(c), m, n, k, group_m);
 }
 
-// BAND is the default band height, in tile rows. Eight blocks of a round run
-// side by side on each XCD, and the band's shape decides how many different
-// panels they read through that XCD's L2. Over 11 shapes of 5 formats against
-// 8 rows: 128x128 takes 3.4 % less with 6 (2.7 % with 4; FP8 2048^3 11.5 ->
-// 11.1 us, 6000x512x2048 10.2 -> 9.2, never over 0.5 % more), 256x128 3.7 %
-// less with 4 (FP8 8192x1024x2048 22.6 -> 19.4 us, BF16 35.8 -> 33.5); the
-// pairs take 1.1 % more with 6 and 64x64 is level, so both keep 8.
+// BAND is the default band height, in tile rows. An XCD takes consecutive
+// tiles, 32 a round where a CU holds one, and the band's shape decides which
+// panels they share in its L2. Over 11 shapes of 5 formats against 8 rows:
+// 128x128 takes 3.4 % less with 6 (2.7 % with 4; FP8 2048^3 11.5 -> 11.1 us,
+// 6000x512x2048 10.2 -> 9.2, never over 0.5 % more), 256x128 3.7 % less with 4
+// (FP8 8192x1024x2048 22.6 -> 19.4 us, BF16 35.8 -> 33.5); the pairs take 1.1 %
+// more with 6 and 64x64 is level, so both keep 8. BF16 2048^3 gains 4 % (20.2 ->
+// 19.4 us) with the same 12 panels an XCD and the same 50 MB of reads over the
+// fabric, by counter: there it is not the bytes, and what it is stays open.
 #define MB_RING(FMT, OP, BM, BN, STAGES, BAND, RESIDENT, COST, NAME)                                     \
   GemmKernel {                                                                                           \
     FMT, BM, BN, BAND, RESIDENT, COST, NAME,                                                             \
