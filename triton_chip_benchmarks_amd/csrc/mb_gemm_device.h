@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "mb_gemm_offsets.h"
 #include "mb_internal.h"
 #include "mb_mfma.h"
 
@@ -41,10 +42,6 @@ __device__ __forceinline__ void band_tile(int tiles_m, int tiles_n, int group_m,
   tile_m = first_m + (pid % band) % rows_in_band;
   tile_n = (pid % band) / rows_in_band;
 }
-
-// A byte offset past every buffer resource (num_records stays below 2^31):
-// loads from it give zeros, stores to it are dropped.
-constexpr int kOutOfRange = static_cast<int>(0x80000000u);
 
 // Tile of workgroup blockIdx.x for any grid size: XCD x (ids x, x+8, ..) owns
 // a contiguous share of the band order, the first count % 8 XCDs one tile more.

@@ -128,11 +128,9 @@ __global__ void __launch_bounds__(256)
     vb[i] = (wave * (BN / 4) + 8 * i + drow) * row_bytes + 16 * ((i & 1) ? chunk1 : chunk0);
   const uint32_t lds_base =
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
-  // Scales: waves 0 and 2 move A's, 128 rows (1 KiB) each, 1 and 3 B's. Tiles
-  // of up to 128 rows are moved twice, so that every wave has the same DMA count.
   const int scale_half = BM > 128 && !(wave & 1) ? wave >> 1 : 0;
   const int scale_rows = (wave & 1) ? N : M;
-  const int scale_row0 = (wave & 1) ? n0 : m0 + scale_half * 128;
+  const int scale_row0 = scale_first_row(BM, wave, m0, n0);
   const __amdgpu_buffer_rsrc_t rs =
       (wave & 1) ? buffer_rsrc(SB, Op::SCALED ? k_steps * N * 8 : 0) : buffer_rsrc(SA, Op::SCALED ? k_steps * M * 8 : 0);
 
@@ -149,8 +147,8 @@ __global__ void __launch_bounds__(256)
       dma16(rb, kb < ((j & 1) ? limit1 : limit0) ? vb[j] : kOutOfRange, soffset,
             lds_base + stage + (BM + wave * (BN / 4) + 8 * j) * ROWB);
     } else {
-      const int at = __builtin_amdgcn_readfirstlane(kt < k_steps ? (kt * scale_rows + scale_row0) * 8 : 0);
-      dma16(rs, kt < k_steps ? lane * 16 : kOutOfRange, at,
+      const DmaOffsets at = scale_offsets(kt, k_steps, scale_rows, scale_row0, lane);
+      dma16(rs, at.lane, __builtin_amdgcn_readfirstlane(at.scalar),
             lds_base + stage + T::OPERANDS + ((wave & 1) ? T::SCALES_A : scale_half * 1024));
     }
   };
