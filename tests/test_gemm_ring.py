@@ -200,3 +200,21 @@ def test_ring_loops_wait_for_every_dma_and_every_read():
                 pending = False
             elif audit.mnemonic(line) == "s_barrier":
                 assert not pending, name
+
+
+def test_lds_dmas_wait_a_state_after_the_write_of_m0():
+    """An LDS-DMA load takes its LDS address from m0: between the scalar write of m0 and the load stands another
+    instruction, in every GEMM kernel."""
+    from triton_chip_benchmarks_amd import _native, audit
+
+    seen = 0
+    for name in _native.kernel_names():
+        if not name.startswith("gemm_") or name.endswith("_checked"):
+            continue
+        body = audit.instructions(name)
+        for before, line in zip(body, body[1:]):
+            if line.split("//")[0].rstrip().endswith(" lds"):
+                seen += 1
+                destination = before.split(",")[0].split()[1:]
+                assert destination != ["m0"], (name, before, line)
+    assert seen > 1000

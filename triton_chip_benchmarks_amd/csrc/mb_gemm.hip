@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(256)
   // Block `block` into ring slot (slot & 3); past the last step the block is
   // clamped but the slot is not, so a slot still being read is never written.
   auto scale_dma = [&](int slot, int block) __attribute__((always_inline)) {
-    dma16(rs, lane * 16, (block * s_rows + s_row0) * 8, scale_lds + (slot & 3) * SCALE_STAGE);
+    dma16(rs, lane * 16, (block * s_rows + s_row0) * 8, scale_lds, (slot & 3) * SCALE_STAGE);
   };
 
   const int wm = wave & 1, wn = wave >> 1;
@@ -540,16 +540,25 @@ __global__ void __launch_bounds__(256)
   for (int i = 0; i < 8; ++i) dvoff[i] = (64 * wave + 8 * i) * row_bytes + ((i & 1) ? dvoff1 : dvoff0);
   const int limit0 = row_bytes - (((lane & 7) ^ (drow >> 1)) << 4);
   const int limit1 = row_bytes - (((lane & 7) ^ ((drow >> 1) | 4)) << 4);
+  auto dma_from = [&](int kt, int i) __attribute__((always_inline)) {
+    if constexpr (RAGGED)
+      return DmaOffsets{kt * ROWB < ((i & 1) ? limit1 : limit0) ? dvoff[i] : kOutOfRange,
+                        __builtin_amdgcn_readfirstlane(kt < k_steps ? kt * ROWB : 0)};
+    else
+      return DmaOffsets{(i & 1) ? dvoff1 : dvoff0, min(kt, last) * ROWB + (64 * wave + 8 * i) * row_bytes};
+  };
+  const uint32_t dma_lds = lds_base + 64 * wave * ROWB;
   auto dma = [&](__amdgpu_buffer_rsrc_t r, int region, int kt, int i) __attribute__((always_inline)) {
-    const int row = 64 * wave + 8 * i;
-    const uint32_t to = lds_base + region * REGION + row * ROWB;
-    if constexpr (RAGGED) {
-      const int kb = kt * ROWB;
-      dma16(r, kb < ((i & 1) ? limit1 : limit0) ? dvoff[i] : kOutOfRange,
-            __builtin_amdgcn_readfirstlane(kt < k_steps ? kb : 0), to);
-    } else {
-      dma16(r, (i & 1) ? dvoff1 : dvoff0, min(kt, last) * ROWB + row * row_bytes, to);
-    }
+    const DmaOffsets from = dma_from(kt, i);
+    dma16(r, from.lane, from.scalar, dma_lds + 8 * i * ROWB, region * REGION);
+  };
+  // In two parts: the address, then, a block update later, the load.
+  auto dma_to = [&](int region, int i) __attribute__((always_inline)) {
+    return dma_address(dma_lds + 8 * i * ROWB, region * REGION);
+  };
+  auto dma_load = [&](uint32_t to, __amdgpu_buffer_rsrc_t r, int kt, int i) __attribute__((always_inline)) {
+    const DmaOffsets from = dma_from(kt, i);
+    dma16_at(to, r, from.lane, from.scalar);
   };
 
   const int wm = wave & 1, wn = wave >> 1;
@@ -620,12 +629,14 @@ __global__ void __launch_bounds__(256)
   int slot = 0;  // A slot of the current step: kt % 3
   auto step = [&](int kt, int s) __attribute__((always_inline)) {
     const int next_slot = slot == 2 ? 0 : slot + 1, prev_slot = slot == 0 ? 2 : slot - 1;
+    uint32_t to = 0;  // LDS address of the next DMA
     static_for<0, 32>([&](auto q_c) __attribute__((always_inline)) {
       constexpr int q = decltype(q_c)::value, i = q / 4, j = 4 + q % 4;
       constexpr int rd = q < 8 && q % 2 == 0 ? q / 2 : -1;
       if constexpr (rd >= 0) fb[rd] = frag_b(s, rd);
+      if constexpr (q % 4 == 0) to = dma_to(prev_slot, q / 4);
       constexpr int da = q % 4 == 1 ? q / 4 : -1;
-      if constexpr (da >= 0) dma(ra, prev_slot, kt + 2, da);
+      if constexpr (da >= 0) dma_load(to, ra, kt + 2, da);
       mma(fa[i], fb[j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -636,8 +647,9 @@ __global__ void __launch_bounds__(256)
       constexpr int q = decltype(q_c)::value, i = q / 4, j = q % 4;
       constexpr int rd = q < 8 && q % 2 == 0 ? 4 + q / 2 : -1;
       if constexpr (rd >= 0) fb[rd] = frag_b(s ^ 1, rd);
+      if constexpr (q % 4 == 0) to = dma_to(3 + s, q / 4);
       constexpr int db = q % 4 == 1 ? q / 4 : -1;
-      if constexpr (db >= 0) dma(rb, 3 + s, kt + 2, db);
+      if constexpr (db >= 0) dma_load(to, rb, kt + 2, db);
       mma(fa[i], fb[j], acc[i][j]);
       if constexpr (j == 3) fa[i] = frag_a(next_slot, i);
       __builtin_amdgcn_sched_barrier(0);
@@ -757,7 +769,7 @@ __global__ void __launch_bounds__(256)
       static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
   auto dma_a = [&](int slot, int kt, int i) __attribute__((always_inline)) {
     const int row = 64 * wave + 8 * i;
-    dma16(ra, (i & 1) ? avoff1 : avoff0, kt * ROWB + row * row_bytes, lds_base + slot * AREG + row * ROWB);
+    dma16(ra, (i & 1) ? avoff1 : avoff0, kt * ROWB + row * row_bytes, lds_base + row * ROWB, slot * AREG);
   };
 
   const int wm = wave & 1, wn = wave >> 1;

@@ -13,14 +13,32 @@ namespace mb {
 
 constexpr int kXcds = 8;
 
-// One 16-byte-per-lane LDS DMA: lane l's 16 bytes land at lds_addr + 16 * l.
-// Issued as inline assembly so the compiler's wait-count pass does not force a
-// full vmcnt(0) before every LDS read; the staged kernel issues it ahead of
-// compiler-visible loads, whose in-order vmcnt waits then cover it.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset, uint32_t lds_addr) {
-  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(rsrc), "s"(soffset),
-               "{m0}"(__builtin_amdgcn_readfirstlane(lds_addr))
+// One 16-byte-per-lane LDS DMA: lane l's 16 bytes land at the LDS address in m0
+// + 16 * l. Issued as inline assembly so the compiler's wait-count pass does not
+// force a full vmcnt(0) before every LDS read; the staged kernel issues it ahead
+// of compiler-visible loads, whose in-order vmcnt waits then cover it.
+//
+// The load needs a wait state after the scalar write of m0, which the compiler
+// puts for its own LDS loads only. dma16 does both, with a wait state. The
+// all-DMA 256x256 kernels' loops, where that costs 1.2% (BF16 8192^3 719 -> 728
+// us), write m0 (dma_address) a block update before the load (dma16_at) instead:
+// 695 us where the write directly before the load takes 701.
+__device__ __forceinline__ uint32_t dma_address(uint32_t lds, uint32_t lds_add) {
+  uint32_t m0;
+  asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(m0) : "s"(lds), "s"(lds_add) : "scc");
+  return m0;
+}
+
+__device__ __forceinline__ void dma16_at(uint32_t m0, __amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(rsrc), "s"(soffset), "{m0}"(m0)
                : "memory");
+}
+
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int voffset, int soffset, uint32_t lds,
+                                      uint32_t lds_add) {
+  asm volatile("s_add_u32 m0, %3, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(rsrc),
+               "s"(soffset), "s"(lds), "s"(lds_add)
+               : "m0", "scc", "memory");
 }
 
 // Word 3 of a gfx9 buffer resource: 32-bit data format, no swizzle, raw offsets.

@@ -141,15 +141,15 @@ __global__ void __launch_bounds__(256)
     const int soffset = __builtin_amdgcn_readfirstlane(kt < k_steps ? kb : 0);  // an offset past num_records would wrap the bounds check
     if constexpr (i < T::DMA_A) {
       dma16(ra, kb < ((i & 1) ? limit1 : limit0) ? va[i] : kOutOfRange, soffset,
-            lds_base + stage + (wave * (BM / 4) + 8 * i) * ROWB);
+            lds_base + (wave * (BM / 4) + 8 * i) * ROWB, stage);
     } else if constexpr (i < T::DMA_A + T::DMA_B) {
       constexpr int j = i - T::DMA_A;
       dma16(rb, kb < ((j & 1) ? limit1 : limit0) ? vb[j] : kOutOfRange, soffset,
-            lds_base + stage + (BM + wave * (BN / 4) + 8 * j) * ROWB);
+            lds_base + (BM + wave * (BN / 4) + 8 * j) * ROWB, stage);
     } else {
       const DmaOffsets at = scale_offsets(kt, k_steps, scale_rows, scale_row0, lane);
       dma16(rs, at.lane, __builtin_amdgcn_readfirstlane(at.scalar),
-            lds_base + stage + T::OPERANDS + ((wave & 1) ? T::SCALES_A : scale_half * 1024));
+            lds_base + T::OPERANDS + ((wave & 1) ? T::SCALES_A : scale_half * 1024), stage);
     }
   };
 
