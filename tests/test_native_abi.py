@@ -123,3 +123,10 @@ def test_vector_kernels_and_host_side_rejections():
     assert library.mb_vector_chains(0, fake, fake, fake, 64, 4, 4, 64, 16, 1 << 20, 64,
                                     None) == _native.MB_ERR_INVALID  # input too small
     assert "too small" in _native.last_error()
+
+
+def test_the_launched_kernel_of_an_invalid_gemm_raises_the_library_message():
+    config = _native.gemm_configs("bf16")[0]
+    with pytest.raises(_native.NativeError, match="16 bytes") as raised:
+        _native.gemm_launched_kernel("bf16", config, 64, 64, 3)
+    assert raised.value.code == _native.MB_ERR_INVALID

@@ -272,7 +272,7 @@ def gemm_launched_kernel(dtype: str, config: dict, m: int, n: int, k: int, scale
     name = load().mb_gemm_launched_kernel(MATRIX_FORMATS[dtype], ctypes.byref(_gemm_config(config)), m, n, k,
                                           _buffer(scale_a)[0], _buffer(scale_b)[0])
     if not name:
-        raise NativeError(last_error())
+        raise NativeError(MB_ERR_INVALID, last_error())
     return name.decode()
 
 
