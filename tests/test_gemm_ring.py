@@ -63,6 +63,22 @@ def test_a_launch_never_exceeds_the_requested_tile(dtype):
         assert _launched(dtype, config, 64, 64, (1 << 22) * CHUNK[dtype]).endswith("_checked")
 
 
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_very_tall_and_wide_shapes_get_a_grid_that_hip_takes(dtype):
+    """A launch may have at most 2^32 - 1 work items, so 2^24 - 1 workgroups of 256: where 64x64 tiles are more, a
+    larger tile runs; where every tile the caller allows is more, the call is refused."""
+    from triton_chip_benchmarks_amd import _native
+
+    config = max(_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"])
+    for m, n in [(2**30, 1), (2**30 + 1, 64), (1, 2**30), (70, 2**29), (2**20, 2**10), (2**30 - 64, 1)]:
+        name = _launched(dtype, config, m, n, CHUNK[dtype])
+        tile_m, tile_n, _ = (int(x) for x in name.split("_")[2].split("x"))
+        assert -(-m // tile_m) * -(-n // tile_n) * 256 < 2**32, (m, n, name)
+    small = {**config, "tile_m": 128, "tile_n": 128}
+    with pytest.raises(_native.NativeError, match="too many tiles"):
+        _launched(dtype, small, 2**31 - 1, 1, CHUNK[dtype])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", FORMATS)
 @pytest.mark.parametrize("m,n,chunks", SHAPES)

@@ -1067,11 +1067,17 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
   const uint64_t row_bytes = row_bits / 8, steps = (row_bytes + 127) / 128;
   const mb_gemm_config& v = variant->config;
 
+  // HIP takes at most 2^32 - 1 work items a launch, 256 of them a workgroup.
+  auto grid_fits = [&](const GemmKernel& kernel) {
+    const uint64_t tiles_m = (static_cast<uint64_t>(m) + kernel.tile_m - 1) / kernel.tile_m;
+    const uint64_t tiles_n = (static_cast<uint64_t>(n) + kernel.tile_n - 1) / kernel.tile_n;
+    return tiles_m * tiles_n <= 0xffffffffull / 256;
+  };
   const GemmKernel* best = nullptr;
   double best_cost = 0;
   auto consider = [&](const GemmKernel& kernel) {
     if (kernel.format != format || kernel.tile_m > static_cast<int>(v.tile_m) ||
-        kernel.tile_n > static_cast<int>(v.tile_n))
+        kernel.tile_n > static_cast<int>(v.tile_n) || !grid_fits(kernel))
       return;
     const double cost = gemm_cost(kernel, m, n, steps);
     if (best == nullptr || cost < best_cost) best = &kernel, best_cost = cost;
@@ -1102,7 +1108,8 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
   for (int i = 0; i < ring_count; ++i) consider_any_shape(ring[i]);
   if (best == nullptr)
     for (const GemmKernel& kernel : kCheckedKernels)
-      if (kernel.format == format) best = &kernel;
+      if (kernel.format == format && grid_fits(kernel)) best = &kernel;
+  if (best == nullptr) return fail(MB_ERR_INVALID, "%s: too many tiles", entry);
   out->variant = variant;
   out->kernel = best;
   return MB_OK;
