@@ -227,6 +227,17 @@ int mb_gemm(int format, const mb_gemm_config* config, const void* a, uint64_t a_
             uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n, uint32_t k,
             uint32_t group_m, void* stream);
 
+/* mb_gemm on a kernel of exactly the configured tile, as a sweep over tiles
+ * measures them, however many CUs that leaves idle. MB_ERR_UNSUPPORTED where no
+ * kernel of the tile takes the shape (256x256 tiles of MXFP4 and FP32 and
+ * 256x128 of FP64 need an even number of at least four whole 128-byte K steps
+ * and whole tiles in M and N).
+ * Replaces: bench_tensor.py:212-246 (_configs, _launch: one launch a tile). */
+int mb_gemm_exact_tile(int format, const mb_gemm_config* config, const void* a, uint64_t a_bytes, const void* b,
+                       uint64_t b_bytes, const void* scale_a, uint64_t scale_a_bytes, const void* scale_b,
+                       uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n, uint32_t k,
+                       uint32_t group_m, void* stream);
+
 /* Registered name of the kernel mb_gemm launches for this call (of the
  * requested tile or a smaller one; "_checked" for rows too long for the fast
  * kernels' 32-bit offsets), for the instruction and resource audit of what actually runs; NULL
@@ -235,6 +246,10 @@ int mb_gemm(int format, const mb_gemm_config* config, const void* a, uint64_t a_
  * (bench_tensor.py:594-600, 988). */
 const char* mb_gemm_launched_kernel(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k,
                                     const void* scale_a, const void* scale_b);
+
+/* The same for mb_gemm_exact_tile. */
+const char* mb_gemm_exact_tile_kernel(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k,
+                                      const void* scale_a, const void* scale_b);
 
 /* ---- vector: register-resident arithmetic chains ------------------------ */
 

@@ -31,11 +31,11 @@ class _Scales:
         return 1
 
 
-def _launched(dtype, config, m, n, k):
+def _launched(dtype, config, m, n, k, **options):
     from triton_chip_benchmarks_amd import _native
 
     scales = (_Scales(), _Scales()) if dtype == "fp4" else (None, None)
-    return _native.gemm_launched_kernel(dtype, config, m, n, k, *scales)
+    return _native.gemm_launched_kernel(dtype, config, m, n, k, *scales, **options)
 
 
 @pytest.mark.parametrize("dtype", FORMATS)
@@ -61,6 +61,46 @@ def test_a_launch_never_exceeds_the_requested_tile(dtype):
             tile_m, tile_n, _ = (int(x) for x in tile.split("x"))
             assert tile_m <= config["tile_m"] and tile_n <= config["tile_n"], (config, m, n, k, tile)
         assert _launched(dtype, config, 64, 64, (1 << 22) * CHUNK[dtype]).endswith("_checked")
+
+
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_an_exact_tile_launch_runs_that_tile_or_is_refused(dtype):
+    """exact_tile: the kernel's tile is the configured one whatever else would be faster; where no kernel of the tile
+    takes the shape the call is refused."""
+    from triton_chip_benchmarks_amd import _native
+
+    step = 8 * CHUNK[dtype]
+    for config in _configs(dtype):
+        for m, n, k in [(512, 768, 4 * step), (2048, 2048, 16 * step), (300, 200, CHUNK[dtype])]:
+            takes_any = config["tile_m"] == config["tile_n"] == 128 or config["tile_n"] < 256 and \
+                not (dtype == "fp64" and config["tile_m"] == 256) or dtype in ("bf16", "fp16", "int8", "fp8")
+            if m == 300 and not takes_any:
+                with pytest.raises(_native.NativeError, match="no kernel of tile"):
+                    _launched(dtype, config, m, n, k, exact_tile=True)
+                continue
+            tile = _native.gemm_kernel_tile(_launched(dtype, config, m, n, k, exact_tile=True))
+            assert {key: tile[key] for key in config} == config, (m, n, k)
+
+
+@pytest.mark.parametrize("dtype", FORMATS)
+@pytest.mark.parametrize("size", [256, 2048, 3000])
+def test_the_gemm_sweep_times_every_tile_on_a_kernel_of_its_own(dtype, size):
+    from triton_chip_benchmarks_amd import _native, gemm
+
+    scales = (_Scales(), _Scales()) if dtype == "fp4" else (None, None)
+    size = -(-size // 32) * 32
+    launches = gemm.sweep_launches(dtype, _configs(dtype), size, scales)
+    names = [name for _, _, name in launches]
+    assert len(set(names)) == len(names)
+    assert _launched(dtype, max(_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"]), size, size, size) in names
+    for config, exact_tile, name in launches:
+        tile = _native.gemm_kernel_tile(name)
+        if exact_tile:
+            assert (tile["tile_m"], tile["tile_n"]) == (config["tile_m"], config["tile_n"])
+    if size == 2048:
+        assert sum(exact for _, exact, _ in launches) == len(_configs(dtype))
+    only = gemm.sweep_launches(dtype, _configs(dtype)[:1], size, scales, automatic=False)
+    assert len(only) == 1
 
 
 @pytest.mark.parametrize("dtype", FORMATS)

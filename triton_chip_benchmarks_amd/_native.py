@@ -107,6 +107,9 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "mb_gemm_launched_kernel": (ctypes.c_char_p, [_i32, ctypes.POINTER(GemmConfig), _u32, _u32, _u32, _ptr, _ptr]),
     "mb_gemm": (_i32, [_i32, ctypes.POINTER(GemmConfig), _ptr, _u64, _ptr, _u64, _ptr, _u64, _ptr, _u64, _ptr, _u64,
                        _u32, _u32, _u32, _u32, _ptr]),
+    "mb_gemm_exact_tile": (_i32, [_i32, ctypes.POINTER(GemmConfig), _ptr, _u64, _ptr, _u64, _ptr, _u64, _ptr, _u64,
+                                  _ptr, _u64, _u32, _u32, _u32, _u32, _ptr]),
+    "mb_gemm_exact_tile_kernel": (ctypes.c_char_p, [_i32, ctypes.POINTER(GemmConfig), _u32, _u32, _u32, _ptr, _ptr]),
     "mb_vector_kernel_name": (ctypes.c_char_p, [_i32, _u32]),
     "mb_vector_chains": (_i32, [_i32, _ptr, _ptr, _ptr, _u64, _u32, _u32, _u32, _u64, _u64, _u64, _ptr]),
 }
@@ -267,25 +270,35 @@ def gemm_kernel_name(dtype: str, config: dict) -> str | None:
     return name.decode() if name else None
 
 
-def gemm_launched_kernel(dtype: str, config: dict, m: int, n: int, k: int, scale_a=None, scale_b=None) -> str:
-    """Registered name of the kernel mb_gemm launches for this shape (fast or checked path)."""
-    name = load().mb_gemm_launched_kernel(MATRIX_FORMATS[dtype], ctypes.byref(_gemm_config(config)), m, n, k,
-                                          _buffer(scale_a)[0], _buffer(scale_b)[0])
+def gemm_launched_kernel(dtype: str, config: dict, m: int, n: int, k: int, scale_a=None, scale_b=None,
+                         exact_tile: bool = False) -> str:
+    """Registered name of the kernel that `gemm` launches for this shape."""
+    query = load().mb_gemm_exact_tile_kernel if exact_tile else load().mb_gemm_launched_kernel
+    name = query(MATRIX_FORMATS[dtype], ctypes.byref(_gemm_config(config)), m, n, k, _buffer(scale_a)[0],
+                 _buffer(scale_b)[0])
     if not name:
         raise NativeError(MB_ERR_INVALID, last_error())
     return name.decode()
 
 
+def gemm_kernel_tile(name: str) -> dict:
+    """The tile of a GEMM kernel's registered name, as in `gemm_configs`."""
+    tile_m, tile_n, tile_k = (int(size) for size in name.split("_")[2].split("x"))
+    return {"tile_m": tile_m, "tile_n": tile_n, "tile_k": tile_k, "threads": 256}
+
+
 def gemm(dtype: str, config: dict, a, b, c, m: int, n: int, k: int, scale_a=None, scale_b=None, group_m: int = 0,
-         stream=None) -> None:
-    """C = A . B^T-stored (both K-contiguous) on the current stream."""
+         stream=None, exact_tile: bool = False) -> None:
+    """C = A . B^T-stored (both K-contiguous) on the current stream, on a kernel of at most the configured tile or,
+    with exact_tile, of exactly that tile."""
     a_ptr, a_bytes = _buffer(a)
     b_ptr, b_bytes = _buffer(b)
     sa_ptr, sa_bytes = _buffer(scale_a)
     sb_ptr, sb_bytes = _buffer(scale_b)
     c_ptr, c_bytes = _buffer(c)
-    call("mb_gemm", MATRIX_FORMATS[dtype], ctypes.byref(_gemm_config(config)), a_ptr, a_bytes, b_ptr, b_bytes,
-         sa_ptr, sa_bytes, sb_ptr, sb_bytes, c_ptr, c_bytes, m, n, k, group_m, stream_handle(stream))
+    call("mb_gemm_exact_tile" if exact_tile else "mb_gemm", MATRIX_FORMATS[dtype], ctypes.byref(_gemm_config(config)),
+         a_ptr, a_bytes, b_ptr, b_bytes, sa_ptr, sa_bytes, sb_ptr, sb_bytes, c_ptr, c_bytes, m, n, k, group_m,
+         stream_handle(stream))
 
 
 def stream_handle(stream=None) -> int | None:

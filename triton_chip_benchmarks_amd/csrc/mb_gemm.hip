@@ -1045,8 +1045,10 @@ struct GemmChoice {
   const GemmKernel* kernel;
 };
 
-int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k, const void* scale_a,
-                const void* scale_b, const char* entry, GemmChoice* out) {
+// `exact`: a kernel of the configured tile only, where a launch otherwise uses
+// any of at most that tile.
+int choose_gemm(int format, const mb_gemm_config* config, bool exact, uint32_t m, uint32_t n, uint32_t k,
+                const void* scale_a, const void* scale_b, const char* entry, GemmChoice* out) {
   if (int rc = matrix_format_check(format, entry)) return rc;
   if (config == nullptr) return fail(MB_ERR_INVALID, "%s: config is NULL", entry);
   const GemmVariant* variant = find_gemm(format, config);
@@ -1073,12 +1075,16 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
     const uint64_t tiles_n = (static_cast<uint64_t>(n) + kernel.tile_n - 1) / kernel.tile_n;
     return tiles_m * tiles_n <= 0xffffffffull / 256;
   };
+  auto same_tile = [&](const GemmKernel& kernel) {
+    return kernel.tile_m == static_cast<int>(v.tile_m) && kernel.tile_n == static_cast<int>(v.tile_n);
+  };
   const GemmKernel* best = nullptr;
   double best_cost = 0;
   auto consider = [&](const GemmKernel& kernel) {
     if (kernel.format != format || kernel.tile_m > static_cast<int>(v.tile_m) ||
         kernel.tile_n > static_cast<int>(v.tile_n) || !grid_fits(kernel))
       return;
+    if (exact && !same_tile(kernel)) return;
     const double cost = gemm_cost(kernel, m, n, steps);
     if (best == nullptr || cost < best_cost) best = &kernel, best_cost = cost;
   };
@@ -1108,11 +1114,47 @@ int choose_gemm(int format, const mb_gemm_config* config, uint32_t m, uint32_t n
   for (int i = 0; i < ring_count; ++i) consider_any_shape(ring[i]);
   if (best == nullptr)
     for (const GemmKernel& kernel : kCheckedKernels)
-      if (kernel.format == format && grid_fits(kernel)) best = &kernel;
+      if (kernel.format == format && grid_fits(kernel) && (!exact || same_tile(kernel))) best = &kernel;
+  if (best == nullptr && exact)
+    return fail(MB_ERR_UNSUPPORTED, "%s: no kernel of tile %ux%ux%u takes %ux%ux%u", entry, v.tile_m, v.tile_n,
+                v.tile_k, m, n, k);
   if (best == nullptr) return fail(MB_ERR_INVALID, "%s: too many tiles", entry);
   out->variant = variant;
   out->kernel = best;
   return MB_OK;
+}
+
+int run_gemm(const char* entry, bool exact, int format, const mb_gemm_config* config, const void* a,
+             uint64_t a_bytes, const void* b, uint64_t b_bytes, const void* scale_a, uint64_t scale_a_bytes,
+             const void* scale_b, uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n,
+             uint32_t k, uint32_t group_m, void* stream) {
+  GemmChoice choice;
+  if (int rc = choose_gemm(format, config, exact, m, n, k, scale_a, scale_b, entry, &choice)) return rc;
+  const GemmVariant* variant = choice.variant;
+  const uint64_t row_bytes = static_cast<uint64_t>(k) * variant->elem_bits / 8;
+  if (a == nullptr || b == nullptr || c == nullptr) return fail(MB_ERR_INVALID, "%s: NULL operand", entry);
+  if (a_bytes < m * row_bytes || b_bytes < n * row_bytes ||
+      c_bytes < static_cast<uint64_t>(m) * n * variant->out_bytes)
+    return fail(MB_ERR_INVALID, "%s: buffers too small for %ux%ux%u", entry, m, n, k);
+  if (!aligned(a, 16) || !aligned(b, 16) || !aligned(c, 16))
+    return fail(MB_ERR_ALIGNMENT, "%s: A, B and C must be 16-byte aligned", entry);
+  if (format == MB_MATRIX_MXFP4) {
+    if (scale_a == nullptr || scale_b == nullptr)
+      return fail(MB_ERR_INVALID, "%s: MXFP4 needs E8M0 scales for A and B", entry);
+    const uint64_t blocks = (k + 255) / 256;
+    if (scale_a_bytes < blocks * m * 8 || scale_b_bytes < blocks * n * 8)
+      return fail(MB_ERR_INVALID, "%s: scale buffers too small ([ceil(K/256)][M|N][8] bytes needed)", entry);
+  }
+  // A band taller than the tile rows acts as the full height, so group_m is
+  // clamped to the row count of the smallest tile a launcher uses: the band's
+  // tile count (group x tile columns) then stays within the int grid.
+  const uint32_t max_group = (m + 63) / 64;
+  const int group = static_cast<int>(group_m ? (group_m < max_group ? group_m : max_group)
+                                             : static_cast<uint32_t>(choice.kernel->default_group));
+  choice.kernel->launch(static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b), static_cast<const uint8_t*>(scale_a),
+                static_cast<const uint8_t*>(scale_b), c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
+                group, static_cast<hipStream_t>(stream));
+  return launch_status(choice.kernel->name);
 }
 
 }  // namespace
@@ -1142,40 +1184,31 @@ int mb_gemm(int format, const mb_gemm_config* config, const void* a, uint64_t a_
             uint64_t b_bytes, const void* scale_a, uint64_t scale_a_bytes, const void* scale_b,
             uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n, uint32_t k,
             uint32_t group_m, void* stream) {
-  using namespace mb;
-  GemmChoice choice;
-  if (int rc = choose_gemm(format, config, m, n, k, scale_a, scale_b, "mb_gemm", &choice)) return rc;
-  const GemmVariant* variant = choice.variant;
-  const uint64_t row_bytes = static_cast<uint64_t>(k) * variant->elem_bits / 8;
-  if (a == nullptr || b == nullptr || c == nullptr) return fail(MB_ERR_INVALID, "mb_gemm: NULL operand");
-  if (a_bytes < m * row_bytes || b_bytes < n * row_bytes ||
-      c_bytes < static_cast<uint64_t>(m) * n * variant->out_bytes)
-    return fail(MB_ERR_INVALID, "mb_gemm: buffers too small for %ux%ux%u", m, n, k);
-  if (!aligned(a, 16) || !aligned(b, 16) || !aligned(c, 16))
-    return fail(MB_ERR_ALIGNMENT, "mb_gemm: A, B and C must be 16-byte aligned");
-  if (format == MB_MATRIX_MXFP4) {
-    if (scale_a == nullptr || scale_b == nullptr)
-      return fail(MB_ERR_INVALID, "mb_gemm: MXFP4 needs E8M0 scales for A and B");
-    const uint64_t blocks = (k + 255) / 256;
-    if (scale_a_bytes < blocks * m * 8 || scale_b_bytes < blocks * n * 8)
-      return fail(MB_ERR_INVALID, "mb_gemm: scale buffers too small ([ceil(K/256)][M|N][8] bytes needed)");
-  }
-  // A band taller than the tile rows acts as the full height, so group_m is
-  // clamped to the row count of the smallest tile a launcher uses: the band's
-  // tile count (group x tile columns) then stays within the int grid.
-  const uint32_t max_group = (m + 63) / 64;
-  const int group = static_cast<int>(group_m ? (group_m < max_group ? group_m : max_group)
-                                             : static_cast<uint32_t>(choice.kernel->default_group));
-  choice.kernel->launch(static_cast<const uint8_t*>(a), static_cast<const uint8_t*>(b), static_cast<const uint8_t*>(scale_a),
-                static_cast<const uint8_t*>(scale_b), c, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
-                group, static_cast<hipStream_t>(stream));
-  return launch_status(choice.kernel->name);
+  return mb::run_gemm("mb_gemm", false, format, config, a, a_bytes, b, b_bytes, scale_a, scale_a_bytes, scale_b,
+                      scale_b_bytes, c, c_bytes, m, n, k, group_m, stream);
+}
+
+int mb_gemm_exact_tile(int format, const mb_gemm_config* config, const void* a, uint64_t a_bytes, const void* b,
+                       uint64_t b_bytes, const void* scale_a, uint64_t scale_a_bytes, const void* scale_b,
+                       uint64_t scale_b_bytes, void* c, uint64_t c_bytes, uint32_t m, uint32_t n, uint32_t k,
+                       uint32_t group_m, void* stream) {
+  return mb::run_gemm("mb_gemm_exact_tile", true, format, config, a, a_bytes, b, b_bytes, scale_a, scale_a_bytes,
+                      scale_b, scale_b_bytes, c, c_bytes, m, n, k, group_m, stream);
 }
 
 const char* mb_gemm_launched_kernel(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k,
                                     const void* scale_a, const void* scale_b) {
   mb::GemmChoice choice;
-  if (mb::choose_gemm(format, config, m, n, k, scale_a, scale_b, "mb_gemm_launched_kernel", &choice)) return nullptr;
+  if (mb::choose_gemm(format, config, false, m, n, k, scale_a, scale_b, "mb_gemm_launched_kernel", &choice))
+    return nullptr;
+  return choice.kernel->name;
+}
+
+const char* mb_gemm_exact_tile_kernel(int format, const mb_gemm_config* config, uint32_t m, uint32_t n, uint32_t k,
+                                      const void* scale_a, const void* scale_b) {
+  mb::GemmChoice choice;
+  if (mb::choose_gemm(format, config, true, m, n, k, scale_a, scale_b, "mb_gemm_exact_tile_kernel", &choice))
+    return nullptr;
   return choice.kernel->name;
 }
 

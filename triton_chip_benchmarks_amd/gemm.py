@@ -2,7 +2,9 @@
 
 Follows the reference's run_gemm (bench_tensor.py:1509-1595): per size and
 tile, validate C against a full-precision reference, then time the kernel and
-report 2*M*N*K operations. Two operand recipes (--inputs):
+report 2*M*N*K operations. Each tile is timed on a kernel of exactly that tile;
+where a call left to choose runs a kernel that is none of these, it gets a row
+of its own. Two operand recipes (--inputs):
 
 baseline (default), the benchmark configuration's GEMM sets:
   bf16/fp16/fp32/fp64  N(0, 1) from the seed; elementwise |C - R| <= atol +
@@ -171,6 +173,28 @@ def validate(c, ref, dtype: str, rows_per_chunk: int = 2048, tolerance: float | 
             "reference": "FP64 torch.matmul on the device (exact for the integer-valued operand sets)"}
 
 
+def sweep_launches(dtype: str, candidates, size: int, scales, automatic: bool = True):
+    """What a sweep at size^3 times, each kernel once: (config given to `gemm`, exact_tile, kernel name) for every
+    candidate tile on a kernel of exactly that tile or, where none of the tile takes the shape, what a call bounded
+    by it runs, and, with `automatic`, for the kernel that a call bounded by the largest tile picks for itself (of a
+    smaller tile where few large ones would leave CUs idle)."""
+    launches = []
+
+    def add(config, exact_tile):
+        kernel = _native.gemm_launched_kernel(dtype, config, size, size, size, *scales, exact_tile=exact_tile)
+        if kernel not in [name for _, _, name in launches]:
+            launches.append((config, exact_tile, kernel))
+
+    for config in candidates:
+        try:
+            add(config, True)
+        except _native.NativeError:
+            add(config, False)
+    if automatic:
+        add(max(_native.gemm_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"]), False)
+    return launches
+
+
 def run_gemm(args, metadata: dict, device) -> None:
     from .bench_tensor import accumulator_name, precision_descriptor, rates
 
@@ -209,13 +233,14 @@ def run_gemm(args, metadata: dict, device) -> None:
         a, b, c, scales, a_values, b_values = gemm_inputs(dtype, size, size, size, device, args.seed, inputs)
         ref = reference(a_values, b_values)
         del a_values, b_values
-        for config in candidates:
-            # The kernel this shape actually launches (a ragged shape runs the tile's checked variant).
-            kernel = _native.gemm_launched_kernel(dtype, config, size, size, size, *(scales or (None, None)))
+        for given, exact_tile, kernel in sweep_launches(dtype, candidates, size, scales or (None, None),
+                                                        not args.tiles):
+            config = _native.gemm_kernel_tile(kernel)
             c.fill_(-2**31 if dtype == "int8" else float("nan"))
 
-            def run(config=config):
-                _native.gemm(dtype, config, a, b, c, size, size, size, *(scales or (None, None)))
+            def run(given=given, exact_tile=exact_tile):
+                _native.gemm(dtype, given, a, b, c, size, size, size, *(scales or (None, None)),
+                             exact_tile=exact_tile)
 
             run()
             torch.cuda.synchronize()
@@ -239,7 +264,7 @@ def run_gemm(args, metadata: dict, device) -> None:
                    **descriptor, **row_rates,
                    "config": {"block_m": config["tile_m"], "block_n": config["tile_n"], "block_k": config["tile_k"],
                               "threads": config["threads"]},
-                   "kernel": kernel, "status": "ok", "correctness": correctness, "compiled": info,
+                   "kernel": kernel, "tile_selection": "exact" if exact_tile else "automatic", "status": "ok", "correctness": correctness, "compiled": info,
                    "roofline": roofline.describe(f"tensor_{dtype}", row_rates["peak_teraops_per_second"]),
                    **timing}
             rows.append(row)
