@@ -328,14 +328,15 @@ class GemmWorkload(Workload):
         self.row, self.label = f"tensor_{dtype}", self.LABELS[dtype]
         self.unit = "TOP/s" if dtype == "int8" else "TFLOP/s"
         self.cfg = max(_native.gemm_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"])
-        self.kernel = _native.gemm_kernel_name(dtype, self.cfg)
         a, b, c, scales, a_values, b_values = gemm.gemm_inputs(dtype, size, size, size, "cuda", GEMM_SEED)
         self.a, self.b, self.c, self.scales = a, b, c, scales or (None, None)
+        self.kernel = _native.gemm_launched_kernel(dtype, self.cfg, size, size, size, *self.scales)
+        tile = _native.gemm_kernel_tile(self.kernel)
         self.reference = gemm.reference(a_values, b_values)
         del a_values, b_values
         self.work = 2 * size**3
-        self.config = {"m": size, "n": size, "k": size, "tile": f"{self.cfg['tile_m']}x{self.cfg['tile_n']}x"
-                       f"{self.cfg['tile_k']}", "layout": "A row-major, B column-major",
+        self.config = {"m": size, "n": size, "k": size, "tile": f"{tile['tile_m']}x{tile['tile_n']}x{tile['tile_k']}",
+                       "layout": "A row-major, B column-major",
                        "operands": gemm.INPUT_PATTERN[dtype], "seed": GEMM_SEED}
 
     def launch(self):
