@@ -1031,11 +1031,18 @@ const GemmVariant* find_gemm(int format, const mb_gemm_config* config) {
 // 256 * resident tiles, then the rest.
 double gemm_cost(const GemmKernel& kernel, uint64_t m, uint64_t n, uint64_t steps) {
   const uint64_t tiles = ((m + kernel.tile_m - 1) / kernel.tile_m) * ((n + kernel.tile_n - 1) / kernel.tile_n);
-  const uint64_t round = 256ull * kernel.resident;
+  const uint64_t round = 256ull * kernel.resident, rounds = tiles / round, rest = tiles % round;
   const GemmCost& cost = kernel.cost;
   auto one = [&](double filled) { return cost.tile + steps * (cost.step_empty + (cost.step_full - cost.step_empty) * filled); };
-  double total = (tiles / round) * one(1.0);
-  if (tiles % round) total += one(static_cast<double>(tiles % round) / round);
+  double total = rounds * one(1.0);
+  if (rest) {
+    double filled = static_cast<double>(rest) / round;
+    if (cost.per_cu) {
+      filled = static_cast<double>((rest + 255) / 256) / kernel.resident;
+      if (rounds) filled = (1.0 + filled) / 2;
+    }
+    total += one(filled);
+  }
   return total;
 }
 

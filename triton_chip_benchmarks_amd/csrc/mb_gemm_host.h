@@ -18,10 +18,14 @@ inline uint32_t tile_count(int m, int n, int bm, int bn) {
 
 // What one round of a kernel's workgroups (`resident` per CU on 256 CUs) takes,
 // in microseconds: `tile` once (prologue, epilogue) and, per 128-byte K step,
-// from `step_empty` to `step_full` with the filled share of the round - operand
-// traffic and the power limit slow a step down as more CUs run.
+// from `step_empty` to `step_full` with the filled share of the round. That is
+// the chip's share where operand traffic and the power limit slow a step down as
+// more CUs run. FP32 (`per_cu`) waits for the matrix cores of the busiest CU:
+// 257 tiles of a pair take as long as 512. After full rounds the rest spreads
+// less evenly, as CUs become free: halfway to a full one.
 struct GemmCost {
   float tile, step_empty, step_full;
+  bool per_cu;
 };
 
 struct GemmKernel {
@@ -39,18 +43,24 @@ struct GemmKernel {
 // BF16, FP8 and MXFP4, which move the same bytes per step and matrix cycle,
 // together). Picking the cheapest estimate costs 0.7% on average against
 // always picking the fastest kernel; always taking the largest tile costs 126%.
-constexpr GemmCost kCost256{7.4f, 0.85f, 1.41f};
-constexpr GemmCost kCost256x128{4.5f, 0.44f, 0.855f};
-constexpr GemmCost kCost128{2.9f, 0.255f, 0.48f};
-constexpr GemmCost kCost128Pair{2.0f, 0.39f, 1.04f};
-constexpr GemmCost kCost64{1.45f, 0.105f, 0.575f};
-constexpr GemmCost kCostF32x256{6.7f, 6.8f, 7.4f};
-constexpr GemmCost kCostF32x128{3.0f, 1.85f, 1.97f};
-constexpr GemmCost kCostF32x128Pair{2.3f, 1.7f, 3.5f};
-constexpr GemmCost kCostF32x64{1.5f, 0.44f, 1.55f};
-constexpr GemmCost kCostF64x256{7.5f, 3.3f, 3.83f};
-constexpr GemmCost kCostF64x128{4.5f, 1.78f, 1.97f};
-constexpr GemmCost kCostF64x64{1.95f, 0.365f, 1.48f};
+constexpr GemmCost kCost256{7.4f, 0.85f, 1.41f, false};
+constexpr GemmCost kCost256x128{4.5f, 0.44f, 0.855f, false};
+constexpr GemmCost kCost128{2.9f, 0.255f, 0.48f, false};
+constexpr GemmCost kCost128Pair{2.0f, 0.39f, 1.04f, false};
+constexpr GemmCost kCost64{1.45f, 0.105f, 0.575f, false};
+// FP32 and FP64, fitted to 545 and 580 shapes (M, N from 128 to 16384, 2 to 512
+// steps, half of them exact) on the kernels that take them: the cheapest estimate
+// costs 0.17% and 0.09% on average against the fastest, at most 10% (19 us) and
+// 5%, and never over 2% more than the largest tile. FP32 8192^3 7432 -> 7166 us,
+// 3072x10240x7744 3607 -> 3402; FP64 512x14848x1856 444 -> 419: a dearer largest
+// tile and, for FP32, the chip's share kept that tile from running.
+constexpr GemmCost kCostF32x256{9.67f, 7.11f, 7.11f, true};
+constexpr GemmCost kCostF32x128{4.71f, 1.974f, 1.974f, true};
+constexpr GemmCost kCostF32x128Pair{4.53f, 0.404f, 3.58f, true};
+constexpr GemmCost kCostF32x64{1.87f, 0.02f, 1.52f, true};
+constexpr GemmCost kCostF64x256{9.5f, 3.6f, 3.7f, false};
+constexpr GemmCost kCostF64x128{5.5f, 1.7f, 1.97f, false};
+constexpr GemmCost kCostF64x64{1.3f, 0.2f, 1.53f, false};
 
 // The ring kernels (mb_gemm_ring.h), compiled in mb_gemm_ring.hip.
 const GemmKernel* ring_kernels(int* count);
