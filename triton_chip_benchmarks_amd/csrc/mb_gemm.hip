@@ -929,7 +929,7 @@ const GemmKernel kExactKernels[] = {
     MB_EXACT(MB_MATRIX_F16, MfmaF16x16, 4, kCost256, "gemm_f16_256x256x64"),
     MB_EXACT(MB_MATRIX_FP8_E4M3, MfmaFp8x16, 6, kCost256, "gemm_fp8_256x256x128"),
     MB_EXACT(MB_MATRIX_I8, MfmaI8x16, 7, kCost256, "gemm_i8_256x256x128"),
-    MB_EXACT(MB_MATRIX_MXFP4, MfmaMxfp4, 8, kCost256, "gemm_mxfp4_256x256x256"),
+    MB_EXACT(MB_MATRIX_MXFP4, MfmaMxfp4, 8, kCostMx256, "gemm_mxfp4_256x256x256"),
     MB_EXACT(MB_MATRIX_F64, MfmaF64, 8, kCostF64x256, "gemm_f64_256x128x16"),
     MB_EXACT(MB_MATRIX_F32, MfmaF32x16, 8, kCostF32x256, "gemm_f32_256x256x32"),
 };

@@ -40,14 +40,23 @@ struct GemmKernel {
 };
 
 // Fitted to 317 launches on an MI355X (M, N from 256 to 8192, 2 to 64 K steps;
-// BF16, FP8 and MXFP4, which move the same bytes per step and matrix cycle,
-// together). Picking the cheapest estimate costs 0.7% on average against
+// BF16, FP8 and MXFP4 together). Picking the cheapest estimate costs 0.7% on average against
 // always picking the fastest kernel; always taking the largest tile costs 126%.
 constexpr GemmCost kCost256{7.4f, 0.85f, 1.41f, false};
 constexpr GemmCost kCost256x128{4.5f, 0.44f, 0.855f, false};
 constexpr GemmCost kCost128{2.9f, 0.255f, 0.48f, false};
 constexpr GemmCost kCost128Pair{2.0f, 0.39f, 1.04f, false};
 constexpr GemmCost kCost64{1.45f, 0.105f, 0.575f, false};
+// MXFP4, whose step is four times the operations of BF16's for the same bytes,
+// fitted to 530 shapes: 0.5% over the fastest on average (the constants above:
+// 1.5% over 350 of them), at most 24% (14 us). Its stages carry scales, so a CU holds two of its 64x64 tiles; priced
+// with three, they ran where 128x128 is faster (8704x256x3584 12.4 us, 128x128
+// 9.6).
+constexpr GemmCost kCostMx256{12.66f, 0.75f, 1.806f, false};
+constexpr GemmCost kCostMx256x128{6.73f, 0.551f, 1.049f, false};
+constexpr GemmCost kCostMx128{4.47f, 0.317f, 0.621f, false};
+constexpr GemmCost kCostMx128Pair{3.63f, 0.661f, 1.247f, false};
+constexpr GemmCost kCostMx64{2.04f, 0.213f, 0.555f, false};
 // FP32 and FP64, fitted to 545 and 580 shapes (M, N from 128 to 16384, 2 to 512
 // steps, half of them exact) on the kernels that take them: the cheapest estimate
 // costs 0.17% and 0.09% on average against the fastest, at most 10% (19 us) and
