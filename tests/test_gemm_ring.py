@@ -187,6 +187,23 @@ def test_kernels_of_any_shape_write_only_c_and_read_nothing_past_their_operands(
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tile", [("fp64", 64), ("fp64", 128), ("fp32", 128)])
+@pytest.mark.parametrize("n", [3101, 3104])
+def test_outputs_of_many_rounds_with_and_without_whole_lines(gpu, dtype, tile, n):
+    """More than two rounds of the chip (2303 tiles of 64x64, 600 of 128x128), with rows of C that share 128-byte
+    lines (n = 3101) and rows of whole lines: the stores take another order and cache policy. A request for 64x64
+    tiles, or for 128x128, which FP32 answers with 64x64 here."""
+    m, k = 3000, 3 * CHUNK[dtype]
+    config = next(c for c in _configs(dtype) if c["tile_m"] == tile)
+    exact = {"exact_tile": True} if dtype == "fp64" else {}
+    name = _launched(dtype, config, m, n, k, **exact)
+    assert name == {64: "gemm_f64_64x64x16", 128: "gemm_f64_128x128x16"}[tile] if exact else "gemm_f32_64x64x32"
+    print(f"gemm {dtype} {m}x{n}x{k} via {name}", flush=True)
+    got, a_values, b_values = _run_gemm(dtype, config, m, n, k, np.random.default_rng(n), **exact)
+    _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp64", "fp8"])
 def test_rows_past_the_32_bit_offsets_run_the_checked_kernel(gpu, dtype):
     """64 rows of 2^25 bytes are the first that a 64x64 tile cannot address with 31-bit offsets."""
@@ -243,6 +260,17 @@ def _ring_kernels():
             _, bm, bn, stages = match.groups()
             out.append((name, int(stages), int(bm) // 32 + int(bn) // 32 + ("mxfp4" in name)))
     return out
+
+
+def test_every_ring_kernel_stores_c_written_through_and_plain():
+    """Written through the L2 (sc1), and plain for outputs of many rounds whose rows share lines, where the former
+    is up to 2.6 times slower (FP64 7072x5406x4 on 64x64 tiles)."""
+    from triton_chip_benchmarks_amd import audit
+
+    for name, _, _ in _ring_kernels():
+        stores = [line.split("//")[0] for line in audit.instructions(name)
+                  if audit.mnemonic(line).startswith("buffer_store_dword")]
+        assert {"sc1" in line for line in stores} == {True, False}, name
 
 
 def test_ring_loops_wait_for_every_dma_and_every_read():

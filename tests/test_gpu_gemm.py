@@ -73,7 +73,7 @@ def _device_operand(torch, values, dtype):
     raise ValueError(dtype)
 
 
-def _run_gemm(dtype, config, m, n, k, rng, normal=False, keep_device=False):
+def _run_gemm(dtype, config, m, n, k, rng, normal=False, keep_device=False, exact_tile=False):
     """Returns (C on the host as float64, A values, B values [n][k]) [+ device C, A, B]."""
     import torch
 
@@ -94,7 +94,7 @@ def _run_gemm(dtype, config, m, n, k, rng, normal=False, keep_device=False):
         a, b = _device_operand(torch, a_values, dtype), _device_operand(torch, b_values, dtype)
     out = torch.int32 if dtype == "int8" else torch.float64 if dtype == "fp64" else torch.float32
     c = torch.full((m, n), -3, dtype=out, device="cuda")
-    _native.gemm(dtype, config, a, b, c, m, n, k, *scales)
+    _native.gemm(dtype, config, a, b, c, m, n, k, *scales, exact_tile=exact_tile)
     torch.cuda.synchronize()
     host = c.cpu().numpy().astype(np.float64)
     if keep_device:

@@ -22,37 +22,31 @@ void launch_ring(const uint8_t* a, const uint8_t* b, const uint8_t* sa, const ui
 // more with 6 and 64x64 is level, so both keep 8. BF16 2048^3 gains 4 % (20.2 ->
 // 19.4 us) with the same 12 panels an XCD and the same 50 MB of reads over the
 // fabric, by counter: there it is not the bytes, and what it is stays open.
-// RESIDENT, the workgroups a CU holds, is bounded by LDS: the kernels take at
-// most 228 (pair) and 108 (64x64) of a SIMD's 512 registers a lane.
-template <class Op, int BM, int BN, int STAGES, int RESIDENT>
-constexpr int resident() {
-  static_assert(RESIDENT * STAGES * RingTile<Op, BM, BN, STAGES>::STAGE <= 160 * 1024, "a CU's LDS");
-  return RESIDENT;
-}
-
-#define MB_RING(FMT, OP, BM, BN, STAGES, BAND, RESIDENT, COST, NAME)                                     \
-  GemmKernel {                                                                                           \
-    FMT, BM, BN, BAND, resident<OP, BM, BN, STAGES, RESIDENT>(), COST, NAME,                             \
+// The workgroups a CU holds are bounded by LDS: the kernels take at most 228
+// (pair) and 108 (64x64) of a SIMD's 512 registers a lane.
+#define MB_RING(FMT, OP, BM, BN, STAGES, BAND, COST, NAME)                                                   \
+  GemmKernel {                                                                                               \
+    FMT, BM, BN, BAND, RingTile<OP, BM, BN, STAGES>::RESIDENT, COST, NAME,                                   \
         reinterpret_cast<const void*>(gemm_ring_kernel<OP, BM, BN, STAGES>), launch_ring<OP, BM, BN, STAGES> \
   }
-#define MB_RING_SET(FMT, OP, TYPE, BK, RESIDENT64, COST)                                        \
-  MB_RING(FMT, OP, 256, 128, 3, 4, 1, COST##256x128, "gemm_" TYPE "_256x128x" BK),              \
-      MB_RING(FMT, OP, 128, 128, 4, 6, 1, COST##128, "gemm_" TYPE "_128x128x" BK),              \
-      MB_RING(FMT, OP, 128, 128, 2, 8, 2, COST##128Pair, "gemm_" TYPE "_128x128x" BK "_pair"),  \
-      MB_RING(FMT, OP, 64, 64, 3, 8, RESIDENT64, COST##64, "gemm_" TYPE "_64x64x" BK)
+#define MB_RING_SET(FMT, OP, TYPE, BK, COST)                                                    \
+  MB_RING(FMT, OP, 256, 128, 3, 4, COST##256x128, "gemm_" TYPE "_256x128x" BK),                 \
+      MB_RING(FMT, OP, 128, 128, 4, 6, COST##128, "gemm_" TYPE "_128x128x" BK),                 \
+      MB_RING(FMT, OP, 128, 128, 2, 8, COST##128Pair, "gemm_" TYPE "_128x128x" BK "_pair"),     \
+      MB_RING(FMT, OP, 64, 64, 3, 8, COST##64, "gemm_" TYPE "_64x64x" BK)
 
 const GemmKernel kRingKernels[] = {
-    MB_RING_SET(MB_MATRIX_BF16, MfmaBf16, "bf16", "64", 3, kCost),
-    MB_RING_SET(MB_MATRIX_F16, MfmaF16, "f16", "64", 3, kCost),
-    MB_RING_SET(MB_MATRIX_FP8_E4M3, MfmaFp8, "fp8", "128", 3, kCost),
-    MB_RING_SET(MB_MATRIX_I8, MfmaI8, "i8", "128", 3, kCost),
-    MB_RING_SET(MB_MATRIX_MXFP4, MfmaMxfp4, "mxfp4", "256", 2, kCostMx),
+    MB_RING_SET(MB_MATRIX_BF16, MfmaBf16, "bf16", "64", kCost),
+    MB_RING_SET(MB_MATRIX_F16, MfmaF16, "f16", "64", kCost),
+    MB_RING_SET(MB_MATRIX_FP8_E4M3, MfmaFp8, "fp8", "128", kCost),
+    MB_RING_SET(MB_MATRIX_I8, MfmaI8, "i8", "128", kCost),
+    MB_RING_SET(MB_MATRIX_MXFP4, MfmaMxfp4, "mxfp4", "256", kCostMx),
     // FP32 and FP64 are bound by the matrix cores at every tile: no 256x128.
-    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 4, 6, 1, kCostF32x128, "gemm_f32_128x128x32"),
-    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 2, 8, 2, kCostF32x128Pair, "gemm_f32_128x128x32_pair"),
-    MB_RING(MB_MATRIX_F32, MfmaF32, 64, 64, 3, 8, 3, kCostF32x64, "gemm_f32_64x64x32"),
-    MB_RING(MB_MATRIX_F64, MfmaF64, 128, 128, 4, 6, 1, kCostF64x128, "gemm_f64_128x128x16"),
-    MB_RING(MB_MATRIX_F64, MfmaF64, 64, 64, 3, 8, 3, kCostF64x64, "gemm_f64_64x64x16"),
+    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 4, 6, kCostF32x128, "gemm_f32_128x128x32"),
+    MB_RING(MB_MATRIX_F32, MfmaF32, 128, 128, 2, 8, kCostF32x128Pair, "gemm_f32_128x128x32_pair"),
+    MB_RING(MB_MATRIX_F32, MfmaF32, 64, 64, 3, 8, kCostF32x64, "gemm_f32_64x64x32"),
+    MB_RING(MB_MATRIX_F64, MfmaF64, 128, 128, 4, 6, kCostF64x128, "gemm_f64_128x128x16"),
+    MB_RING(MB_MATRIX_F64, MfmaF64, 64, 64, 3, 8, kCostF64x64, "gemm_f64_64x64x16"),
 };
 
 struct RingRegistrar {
