@@ -102,6 +102,28 @@ def _run_gemm(dtype, config, m, n, k, rng, normal=False, keep_device=False, exac
     return host, a_values, b_values
 
 
+def _aligned_scales(dtype):
+    """Scale arguments for a question about the dispatch, which looks at their alignment only."""
+    import torch
+
+    return (torch.empty(16, dtype=torch.uint8, device="cuda"),) * 2 if dtype == "fp4" else (None, None)
+
+
+def _takes_tile(dtype, config, m, n, k):
+    """Whether a kernel of exactly the configured tile takes the shape, so that a launch can ask for it (an ordinary
+    one takes the fastest of at most that tile)."""
+    from triton_chip_benchmarks_amd import _native
+
+    try:
+        name = _native.gemm_launched_kernel(dtype, config, m, n, k, *_aligned_scales(dtype), exact_tile=True)
+    except _native.NativeError:
+        return False
+    tile = _native.gemm_kernel_tile(name)
+    assert (tile["tile_m"], tile["tile_n"]) == (config["tile_m"], config["tile_n"])
+    print(f"gemm {dtype} {m}x{n}x{k} via {name}", flush=True)
+    return True
+
+
 def _assert_matches(dtype, got, reference, normal=False):
     if normal or dtype == "fp64":
         ot.check_gemm(got, reference, dtype)
@@ -121,28 +143,28 @@ def test_gemm_matches_oracle_every_tile_and_ragged_shapes(gpu, dtype):
         for m, n, k in shapes:
             print(f"gemm {dtype} tile {config['tile_m']}x{config['tile_n']}x{config['tile_k']} shape {m}x{n}x{k}",
                   flush=True)
-            got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng)
+            got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng,
+                                                exact_tile=_takes_tile(dtype, config, m, n, k))
             _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
 
 
-@pytest.mark.parametrize("dtype", ["bf16", "fp16", "int8", "fp8", "fp32", "fp64"])
+@pytest.mark.parametrize("dtype", FORMATS)
 def test_fast_path_over_step_counts(gpu, dtype):
-    """The fast path (256x256 with A and B by LDS-DMA into rings of three and
-    two slots; 256x128 for FP64, B through registers) at K step counts 4, 6,
-    10, 12 and 14, which wrap the three-slot ring at every phase, on lattice
-    operands (exact; FP64 on N(0,1) within its tolerance), with M != N so a
-    transposed tile order would show."""
+    """The exact-shape kernel of every format (256x256 with A and B by LDS-DMA into rings of three and two slots;
+    256x128 for FP64, B through registers; MXFP4 staged through registers, its scales in a ring of four) at K step
+    counts from 4 to 16, which wrap the rings at every phase, on lattice operands (exact; FP64 on N(0,1) within its
+    tolerance), with M != N so a transposed tile order would show. Such small outputs run on smaller tiles unless the
+    tile is asked for."""
     from triton_chip_benchmarks_amd import _native
 
     rng = np.random.default_rng(23)
     config = max(_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"])
-    elements_per_step = 128 * 8 // {"bf16": 16, "fp16": 16, "int8": 8, "fp8": 8, "fp32": 32, "fp64": 64}[dtype]
-    for steps in (4, 6, 10, 12, 14):
-        m, n, k = 512, 768, steps * elements_per_step
-        launched = _native.gemm_launched_kernel(dtype, config, m, n, k)
-        assert not launched.endswith("_checked"), launched
+    for steps in (4, 6, 8, 10, 12, 14, 16):
+        m, n, k = 512, 768, steps * config["tile_k"]
+        launched = _native.gemm_launched_kernel(dtype, config, m, n, k, *_aligned_scales(dtype), exact_tile=True)
+        assert launched == _native.gemm_kernel_name(dtype, config)
         print(f"gemm {dtype} fast path {m}x{n}x{k} ({steps} K steps) via {launched}", flush=True)
-        got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng)
+        got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng, exact_tile=True)
         _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
 
 
@@ -150,23 +172,75 @@ def test_fast_path_over_step_counts(gpu, dtype):
 def test_band_height_orders_tiles_only(gpu, dtype):
     """group_m orders the tiles and nothing else: every band height, including
     ones taller than the tile rows and values near 2^32 (clamped by mb_gemm),
-    gives the same C on the fast path and on the checked path (ragged shape)."""
+    gives the same C on every tile, with several tile rows and columns of whole
+    tiles and, where a kernel takes them, of a ragged shape."""
     import torch
 
     from triton_chip_benchmarks_amd import _native
 
     rng = np.random.default_rng(31)
+    for config in _configs(dtype):
+        for m, n, k in ((768, 512, 1024), (3 * config["tile_m"] - 60, 3 * config["tile_n"] - 40,
+                                           2 * config["tile_k"])):
+            if not _takes_tile(dtype, config, m, n, k):
+                assert m != 768
+                continue
+            got, a_values, b_values, (c, a, b) = _run_gemm(dtype, config, m, n, k, rng, keep_device=True,
+                                                           exact_tile=True)
+            _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
+            for group in (1, 2, 3, 7, 64, 2**31 + 5, 2**32 - 1):
+                c.fill_(-3)
+                _native.gemm(dtype, config, a, b, c, m, n, k, group_m=group, exact_tile=True)
+                torch.cuda.synchronize()
+                assert np.array_equal(c.cpu().numpy().astype(np.float64), got), group
+
+
+@pytest.mark.parametrize("dtype", FORMATS)
+def test_checked_kernel_over_several_tiles(gpu, dtype):
+    """The kernel of 64-bit addresses, which takes outputs whose 64 rows exceed 31-bit offsets, over two tile rows and
+    2^16 (FP64 2^15) tile columns and several band heights. B repeats a prime number of rows, so the oracle's product
+    of those gives every column, and a tile at a wrong place would show."""
+    import torch
+
+    from triton_chip_benchmarks_amd import _native
+
+    rng = np.random.default_rng(41)
     config = max(_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"])
-    for m, n, k in ((768, 512, 1024), (320, 448, 2 * config["tile_k"])):
-        launched = _native.gemm_launched_kernel(dtype, config, m, n, k)
-        print(f"gemm {dtype} band heights {m}x{n}x{k} via {launched}", flush=True)
-        got, a_values, b_values, (c, a, b) = _run_gemm(dtype, config, m, n, k, rng, keep_device=True)
-        _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T))
-        for group in (1, 2, 3, 7, 64, 2**31 + 5, 2**32 - 1):
-            c.fill_(-3)
-            _native.gemm(dtype, config, a, b, c, m, n, k, group_m=group)
-            torch.cuda.synchronize()
-            assert np.array_equal(c.cpu().numpy().astype(np.float64), got), group
+    period, m = 9973, 130
+    n = (1 << (22 if dtype == "fp64" else 23)) + 77
+    k = {"bf16": 24, "fp16": 24, "fp32": 12, "fp64": 6, "int8": 48, "fp8": 48, "fp4": 96}[dtype]
+    name = _native.gemm_launched_kernel(dtype, config, m, n, k, *_aligned_scales(dtype))
+    assert name.endswith("_checked")
+    scales = (None, None)
+    if dtype == "fp4":
+        codes = [rng.integers(0, 16, (rows, k), dtype=np.uint8) for rows in (m, period)]
+        exponents = [rng.integers(126, 129, (rows, k // 32), dtype=np.uint8) for rows in (m, period)]
+        a_values, b_values = (ot.e2m1_decode(c) * np.repeat(ot.e8m0_decode(e), 32, axis=1)
+                              for c, e in zip(codes, exponents))
+        a, b = (torch.from_numpy(ot.pack_e2m1(c)).cuda() for c in codes)
+        scales = tuple(torch.from_numpy(_scale_blocks(e)).cuda() for e in exponents)
+    else:
+        a_values, b_values = _operand_values(rng, dtype, m, k), _operand_values(rng, dtype, period, k)
+        a, b = _device_operand(torch, a_values, dtype), _device_operand(torch, b_values, dtype)
+    column = torch.arange(n, device="cuda") % period
+    b = b.view(torch.uint8)[column]
+    if dtype == "fp4":
+        scales = (scales[0], scales[1][:, column].contiguous())
+    reference = ot.gemm_reference(a_values, b_values.T)
+    out = torch.int32 if dtype == "int8" else torch.float64 if dtype == "fp64" else torch.float32
+    c = torch.empty((m, n), dtype=out, device="cuda")
+    first = None
+    for group in (0, 1, 2, 64):
+        c.fill_(-3)
+        print(f"gemm {dtype} {m}x{n}x{k} via {name}, bands of {group}", flush=True)
+        _native.gemm(dtype, config, a, b, c, m, n, k, *scales, group_m=group)
+        torch.cuda.synchronize()
+        if first is None:
+            first = c[:, :period].clone()
+            _assert_matches(dtype, first.cpu().numpy().astype(np.float64), reference)
+        for start in range(0, n, 64 * period):
+            part = c[:, start:start + 64 * period]
+            assert torch.equal(part, first.repeat(1, 64)[:, :part.shape[1]]), (group, start)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
@@ -178,7 +252,8 @@ def test_gemm_normal_operands_every_tile_elementwise(gpu, dtype):
                         (config["tile_m"] + 37, config["tile_n"] - 5, 1000)]:
             print(f"gemm {dtype} N(0,1) tile {config['tile_m']}x{config['tile_n']}x{config['tile_k']} "
                   f"shape {m}x{n}x{k}", flush=True)
-            got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng, normal=True)
+            got, a_values, b_values = _run_gemm(dtype, config, m, n, k, rng, normal=True,
+                                                exact_tile=_takes_tile(dtype, config, m, n, k))
             _assert_matches(dtype, got, ot.gemm_reference(a_values, b_values.T), normal=True)
 
 
@@ -189,9 +264,11 @@ def test_gemm_baseline_size_checksums(gpu, dtype, size, normal):
     """Benchmark sizes: row/column checksums, sampled rows against the oracle, and every entry
     against the product's float64 device check. Lattice operands (normal=False) must match
     exactly; N(0,1) operands within the elementwise tolerance."""
-    from triton_chip_benchmarks_amd import gemm
+    from triton_chip_benchmarks_amd import _native, gemm
 
     config = max(_configs(dtype), key=lambda c: c["tile_m"] * c["tile_n"])
+    assert _native.gemm_launched_kernel(dtype, config, size, size, size, *_aligned_scales(dtype)) == \
+        _native.gemm_kernel_name(dtype, config)
     print(f"gemm {dtype} {size}^3 {'N(0,1)' if normal else 'lattice'} "
           f"tile {config['tile_m']}x{config['tile_n']}x{config['tile_k']}", flush=True)
     rng = np.random.default_rng(size + normal)
@@ -225,17 +302,22 @@ def test_mxfp4_gemm_applies_each_rows_group_scale(gpu):
     wrong row or group index, or a scale applied to the wrong operand, moves
     the result off the exact oracle. Products are multiples of 2^-4 below 145
     and K <= 4096, so every partial sum is exact in fp32 in any order. The
-    scales are passed in mb_gemm's K-step block layout; shapes cover the fast
-    path (>= 4 even K steps) and the checked one (2 steps, ragged M/N/K)."""
+    scales are passed in mb_gemm's K-step block layout; every tile runs, the
+    staged 256x256 kernel at step counts that wrap its ring of four scale
+    stages, the others also at a ragged shape (for 256x128 tiles one whose
+    second 128 scale rows lie past M)."""
     import torch
 
     from triton_chip_benchmarks_amd import _native
 
     rng = np.random.default_rng(11)
+    launched = set()
     for config in _configs("fp4"):
         shapes = [(config["tile_m"], config["tile_n"], 2 * config["tile_k"]),
                   (2 * config["tile_m"], config["tile_n"], 4 * config["tile_k"]),
+                  (config["tile_m"], 2 * config["tile_n"], 1536),
                   (config["tile_m"], 2 * config["tile_n"], 2048),
+                  (config["tile_m"], 2 * config["tile_n"], 2560),
                   (config["tile_m"] + 37, config["tile_n"] - 5, 160)]
         for m, n, k in shapes:
             print(f"gemm fp4 scaled tile {config['tile_m']}x{config['tile_n']}x{config['tile_k']} shape {m}x{n}x{k}",
@@ -245,15 +327,18 @@ def test_mxfp4_gemm_applies_each_rows_group_scale(gpu):
             sa = rng.integers(126, 129, (m, k // 32), dtype=np.uint8)
             sb = rng.integers(126, 129, (n, k // 32), dtype=np.uint8)
             c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+            scales = torch.from_numpy(_scale_blocks(sa)).cuda(), torch.from_numpy(_scale_blocks(sb)).cuda()
+            exact_tile = _takes_tile("fp4", config, m, n, k)
+            launched.add(_native.gemm_launched_kernel("fp4", config, m, n, k, *scales, exact_tile=exact_tile))
             _native.gemm("fp4", config, torch.from_numpy(ot.pack_e2m1(codes_a)).cuda(),
-                         torch.from_numpy(ot.pack_e2m1(codes_b)).cuda(), c, m, n, k,
-                         torch.from_numpy(_scale_blocks(sa)).cuda(), torch.from_numpy(_scale_blocks(sb)).cuda())
+                         torch.from_numpy(ot.pack_e2m1(codes_b)).cuda(), c, m, n, k, *scales, exact_tile=exact_tile)
             torch.cuda.synchronize()
             a_values = ot.e2m1_decode(codes_a) * np.repeat(ot.e8m0_decode(sa), 32, axis=1)
             b_values = ot.e2m1_decode(codes_b) * np.repeat(ot.e8m0_decode(sb), 32, axis=1)
             expected = ot.gemm_reference(a_values, b_values.T)
             got = c.cpu().numpy().astype(np.float64)
             assert np.array_equal(got, expected), f"max error {np.abs(got - expected).max()}"
+    assert {_native.gemm_kernel_name("fp4", config) for config in _configs("fp4")} <= launched
 
 
 def test_mxfp4_gemm_reads_the_block_scale_layout_not_row_major(gpu):
@@ -271,6 +356,7 @@ def test_mxfp4_gemm_reads_the_block_scale_layout_not_row_major(gpu):
     config = max(_configs("fp4"), key=lambda c: c["tile_m"] * c["tile_n"])
     m, n, k = config["tile_m"], config["tile_n"], 4 * 256
     print(f"gemm fp4 scale layout {m}x{n}x{k}", flush=True)
+    assert _takes_tile("fp4", config, m, n, k)
     codes_a = rng.integers(0, 16, (m, k), dtype=np.uint8)
     codes_b = rng.integers(0, 16, (n, k), dtype=np.uint8)
     sa = rng.integers(126, 129, (m, k // 32), dtype=np.uint8)
@@ -286,7 +372,8 @@ def test_mxfp4_gemm_reads_the_block_scale_layout_not_row_major(gpu):
         return np.ascontiguousarray(blocks.transpose(1, 0, 2)).reshape(blocks.shape[1], -1)
 
     c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
-    _native.gemm("fp4", config, a, b, c, m, n, k, torch.from_numpy(sa).cuda(), torch.from_numpy(sb).cuda())
+    _native.gemm("fp4", config, a, b, c, m, n, k, torch.from_numpy(sa).cuda(), torch.from_numpy(sb).cuda(),
+                 exact_tile=True)
     torch.cuda.synchronize()
     got = c.cpu().numpy().astype(np.float64)
     misread = product(as_rows(sa.reshape(k // 256, m, 8)), as_rows(sb.reshape(k // 256, n, 8)))
@@ -309,7 +396,7 @@ def test_reference_recipe_ragged_shape_matches_oracle(gpu, dtype):
               f"shape {m}x{n}x{k}", flush=True)
         a, b, c, _scales, a_values, b_values = gemm.gemm_inputs(dtype, m, n, k, "cuda", 9, inputs="reference")
         c.fill_(-3)
-        _native.gemm(dtype, config, a, b, c, m, n, k)
+        _native.gemm(dtype, config, a, b, c, m, n, k, exact_tile=_takes_tile(dtype, config, m, n, k))
         torch.cuda.synchronize()
         got = c.cpu().numpy().astype(np.float64)
         expected = ot.gemm_reference(a_values.cpu().numpy(), b_values.cpu().numpy().T)
