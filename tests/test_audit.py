@@ -112,8 +112,8 @@ def test_registered_names_follow_the_mangled_template_arguments():
     assert audit.registered_name(symbol) == "tensor_peak_bf16_128x128x64_c2_kn"
     assert audit.registered_name("_ZN2mb12_GLOBAL__N_111gemm_kernelINS_9MfmaMxfp4ELi128ELi128ELi256ELi2ELi2ELb1EEEv") \
         == "gemm_mxfp4_128x128x256_checked"
-    assert audit.registered_name("_ZN2mb12_GLOBAL__N_111copy_kernelIDv4_jLi1ELi1EEEv") == "copy_dwordx4_vpt1_nt"
-    assert audit.registered_name("_ZN2mb12_GLOBAL__N_111copy_kernelIjLi8ELi2EEEv") == "copy_dword_vpt8_stream"
+    assert audit.registered_name("_ZN2mb12_GLOBAL__N_111copy_kernelILi1ELi1EEEv") == "copy_dwordx4_vpt1_nt"
+    assert audit.registered_name("_ZN2mb12_GLOBAL__N_117copy_edges_kernelILi8ELi2EEEv") == "copy_edges_vpt8_stream"
     assert audit.registered_name("_ZN2mb12_GLOBAL__N_118gemm_staged_kernelINS_9MfmaMxfp4EEEvPKh") \
         == "gemm_mxfp4_256x256x256"
     assert audit.registered_name("_ZN2mb12_GLOBAL__N_115gemm_dma_kernelINS_11MfmaBf16x16EEEvPKh") \

@@ -13,7 +13,7 @@ import pytest
 
 from triton_chip_benchmarks_amd import counters
 
-COPY = ("void mb::(anonymous namespace)::copy_kernel<unsigned int __vector(4), 1, 2>"
+COPY = ("void mb::(anonymous namespace)::copy_kernel<1, 2>"
         "(unsigned int __vector(4) const*, unsigned int __vector(4)*, unsigned long)")
 GEMM = ("void mb::(anonymous namespace)::gemm_dma_kernel<mb::MfmaBf16x16>(unsigned char const*, "
         "unsigned char const*, unsigned char const*, unsigned char const*, mb::MfmaBf16x16::Out*, int, int, int, int)")
@@ -46,8 +46,8 @@ def test_registered_names_of_demangled_kernels():
         "void mb::(anonymous namespace)::tensor_peak_kernel<mb::MfmaBf16x16, 128, 128, 64, 2, 2, 2, true>"
         "(unsigned char const*)") == "tensor_peak_bf16_128x128x64_c2_mfma16_nk"
     assert counters.registered_name(
-        "void mb::(anonymous namespace)::gemm_kernel<mb::MfmaF64, 64, 64, 16, 2, 2, true>(int)") == \
-        "gemm_f64_64x64x16_checked"
+        "void mb::(anonymous namespace)::gemm_kernel<mb::MfmaF64, 128, 128, 16, 2, 2>(int)") == \
+        "gemm_f64_128x128x16_checked"
     assert counters.registered_name("void mb::(anonymous namespace)::vector_dot4_kernel<16>(int const*)") == \
         "vector_dot4_u16"
     assert counters.registered_name("Cijk_Alik_Bljk_BBS_BH(int)") == "Cijk_Alik_Bljk_BBS_BH"

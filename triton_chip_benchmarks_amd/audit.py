@@ -32,12 +32,11 @@ _GEMM_RE = re.compile(r"gemm_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)ELi(
 _GEMM_RING_RE = re.compile(r"gemm_ring_kernelINS_\d+(Mfma\w+?)ELi(\d+)ELi(\d+)ELi(\d+)EE")
 _GEMM_STAGED_RE = re.compile(r"gemm_(?:staged|dma)_kernelINS_\d+(Mfma\w+?)E(?:Lb([01])E)?E")
 _ELEM_BITS = {"bf16": 16, "f16": 16, "i8": 8, "fp8": 8, "mxfp4": 4, "f32": 32, "f64": 64}
-_COPY_RE = re.compile(r"copy_kernelI(Dv4_j|j|h)Li(\d+)ELi([012])E")
+_COPY_RE = re.compile(r"copy_kernelILi(\d+)ELi([012])E")
 _COPY_EDGES_RE = re.compile(r"copy_edges_kernelILi(\d+)ELi([012])E")
-_READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)Li(\d+)E")
+_READ_RE = re.compile(r"read_sum_kernelI(f|DF16_|t)E")
 _READ_PACKED_RE = re.compile(r"read_sum_packed_kernelI(f|DF16_|t)Li(\d+)E")
 _VECTOR_RE = re.compile(r"vector_(\w+?)_kernelILi(\d+)E")
-_COPY_UNIT = {"Dv4_j": "dwordx4", "j": "dword", "h": "byte"}
 _READ_TYPE = {"f": "f32", "DF16_": "f16", "t": "bf16"}
 
 
@@ -71,8 +70,8 @@ def registered_name(symbol: str) -> str | None:
         return "gemm_f64_256x128x16"
     match = _COPY_RE.search(symbol)
     if match:
-        unit, vpt, policy = match.groups()
-        return f"copy_{_COPY_UNIT[unit]}_vpt{vpt}{('', '_nt', '_stream')[int(policy)]}"
+        vpt, policy = match.groups()
+        return f"copy_dwordx4_vpt{vpt}{('', '_nt', '_stream')[int(policy)]}"
     match = _COPY_EDGES_RE.search(symbol)
     if match:
         vpt, policy = match.groups()

@@ -136,9 +136,7 @@ def registered_name(demangled: str) -> str:
     if family == "gemm_dma_f64_kernel":
         return "gemm_f64_256x128x16"
     if family == "copy_kernel":
-        unit = "dwordx4" if "__vector(4)" in args[0] else "byte" if "char" in args[0] else "dword"
-        policy = {"0": "", "false": "", "1": "_nt", "true": "_nt", "2": "_stream"}[args[2]]
-        return f"copy_{unit}_vpt{args[1]}{policy}"
+        return f"copy_dwordx4_vpt{args[0]}{('', '_nt', '_stream')[int(args[1])]}"
     if family == "copy_edges_kernel":
         return f"copy_edges_vpt{args[0]}{('', '_nt', '_stream')[int(args[1])]}"
     if family in ("read_sum_kernel", "read_sum_packed_kernel"):

@@ -688,15 +688,15 @@ __global__ void __launch_bounds__(256)
         }
   } else {
 #pragma unroll
-  for (int i = 0; i < TILES; ++i)
+    for (int i = 0; i < TILES; ++i)
 #pragma unroll
-    for (int j = 0; j < TILES; ++j)
+      for (int j = 0; j < TILES; ++j)
 #pragma unroll
-      for (int r = 0; r < Op::ACC_REGS; ++r) {
-        const int row = m0 + wm * 128 + i * Op::M + Op::out_row(lane, r);
-        const int col = n0 + wn * 128 + j * Op::N + lrow;
-        C[static_cast<int64_t>(row) * N + col] = acc[i][j][r];
-      }
+        for (int r = 0; r < Op::ACC_REGS; ++r) {
+          const int row = m0 + wm * 128 + i * Op::M + Op::out_row(lane, r);
+          const int col = n0 + wn * 128 + j * Op::N + lrow;
+          C[static_cast<int64_t>(row) * N + col] = acc[i][j][r];
+        }
   }
 #endif
 }

@@ -95,9 +95,8 @@ __device__ __forceinline__ void copy_vectors(const u32x4* __restrict__ src, u32x
   }
 }
 
-// T is the access unit (u32x4); n counts units.
-template <typename T, int VPT, int POLICY>
-__global__ void __launch_bounds__(1024) copy_kernel(const T* __restrict__ src, T* __restrict__ dst,
+template <int VPT, int POLICY>
+__global__ void __launch_bounds__(1024) copy_kernel(const u32x4* __restrict__ src, u32x4* __restrict__ dst,
                                                      uint64_t n) {
   copy_vectors<VPT, POLICY, false>(src, dst, n, blockDim.x);
 }
@@ -159,7 +158,7 @@ __device__ __forceinline__ float to_float<uint16_t>(uint16_t bits) {  // bfloat1
 }
 
 // Sum of one 16-byte vector: four floats, or eight halves, as pairwise sums.
-template <typename T, int VEC>
+template <typename T>
 __device__ __forceinline__ float vector_sum(u32x4 raw) {
   if constexpr (sizeof(T) == 4) {
     const f32x4 v = __builtin_bit_cast(f32x4, raw);
@@ -190,7 +189,7 @@ __device__ __forceinline__ void load_and_sum(float (&value)[N], const T* ptr, bo
   if (serial) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      value[j] = vector_sum<T, VEC>(load_vector(ptr + j * 64 * VEC));
+      value[j] = vector_sum<T>(load_vector(ptr + j * 64 * VEC));
       asm volatile("" : "+v"(ptr) : "v"(value[j]));  // the next address waits for this sum
     }
   } else {
@@ -198,7 +197,7 @@ __device__ __forceinline__ void load_and_sum(float (&value)[N], const T* ptr, bo
 #pragma unroll
     for (int j = 0; j < N; ++j) raw[j] = load_vector(ptr + j * 64 * VEC);
 #pragma unroll
-    for (int j = 0; j < N; ++j) value[j] = vector_sum<T, VEC>(raw[j]);
+    for (int j = 0; j < N; ++j) value[j] = vector_sum<T>(raw[j]);
   }
 }
 
@@ -215,7 +214,7 @@ __device__ __forceinline__ float clipped_sum(const T* base, uint32_t count, uint
     for (uint32_t j = 0; j < 8; ++j)
       raw[j] = p + j * 64 < vectors ? load_vector(base + (p + j * 64) * VEC) : u32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] += vector_sum<T, VEC>(raw[j]);
+    for (int j = 0; j < 8; ++j) acc[j] += vector_sum<T>(raw[j]);
   }
   if (lane < count % VEC) acc[0] += to_float(base[vectors * VEC + lane]);
   return wave_sum(((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
@@ -275,7 +274,7 @@ __global__ void __launch_bounds__(1024)
       const uint32_t vectors = static_cast<uint32_t>(whole - first) * V;
 #pragma unroll
       for (int j = 0; j < LOADS; ++j)
-        value[j] = j * 64 + lane < vectors ? vector_sum<T, VEC>(load_vector(base + j * 64 * VEC)) : 0.f;
+        value[j] = j * 64 + lane < vectors ? vector_sum<T>(load_vector(base + j * 64 * VEC)) : 0.f;
     }
     // One value per segment: pairwise over its loads.
 #pragma unroll
@@ -314,11 +313,11 @@ __global__ void __launch_bounds__(1024)
 
 // Segments of more than kPackedVectors 16-byte vectors: one wave per segment; waves stride
 // over the segments of the buffer.
-template <typename T, int VEC>
+template <typename T>
 __global__ void __launch_bounds__(1024) read_sum_kernel(const T* __restrict__ src, float* __restrict__ sink,
                                                          uint64_t elements, uint32_t block_elements,
                                                          uint64_t segments, bool serial) {
-  static_assert(VEC * sizeof(T) == 16, "16-byte loads");
+  constexpr int VEC = 16 / sizeof(T);
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t waves_per_block = blockDim.x >> 6;
   const uint64_t wave = blockIdx.x * waves_per_block + (threadIdx.x >> 6);
@@ -352,8 +351,8 @@ template <int VPT, int POLICY>
 void launch_copy_kernel(const char* src, char* dst, uint64_t vectors, uint32_t head, uint32_t tail, dim3 grid,
                         dim3 threads, hipStream_t stream) {
   if (head == 0 && tail == 0 && aligned(src, 16))
-    copy_kernel<u32x4, VPT, POLICY><<<grid, threads, 0, stream>>>(reinterpret_cast<const u32x4*>(src),
-                                                                  reinterpret_cast<u32x4*>(dst), vectors);
+    copy_kernel<VPT, POLICY><<<grid, threads, 0, stream>>>(reinterpret_cast<const u32x4*>(src),
+                                                           reinterpret_cast<u32x4*>(dst), vectors);
   else
     copy_edges_kernel<VPT, POLICY><<<grid, threads, 0, stream>>>(reinterpret_cast<const uint8_t*>(src),
                                                                  reinterpret_cast<uint8_t*>(dst), vectors, head, tail);
@@ -381,11 +380,11 @@ int launch_copy(const char* src, char* dst, uint64_t vectors, uint32_t head, uin
 }
 
 #define MB_REGISTER_COPY(P, SUFFIX)                                                         \
-  MB_REGISTER_KERNEL("copy_dwordx4_vpt1" SUFFIX, (copy_kernel<u32x4, 1, P>));               \
-  MB_REGISTER_KERNEL("copy_dwordx4_vpt2" SUFFIX, (copy_kernel<u32x4, 2, P>));               \
-  MB_REGISTER_KERNEL("copy_dwordx4_vpt4" SUFFIX, (copy_kernel<u32x4, 4, P>));               \
-  MB_REGISTER_KERNEL("copy_dwordx4_vpt8" SUFFIX, (copy_kernel<u32x4, 8, P>));               \
-  MB_REGISTER_KERNEL("copy_dwordx4_vpt16" SUFFIX, (copy_kernel<u32x4, 16, P>));             \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt1" SUFFIX, (copy_kernel<1, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt2" SUFFIX, (copy_kernel<2, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt4" SUFFIX, (copy_kernel<4, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt8" SUFFIX, (copy_kernel<8, P>));               \
+  MB_REGISTER_KERNEL("copy_dwordx4_vpt16" SUFFIX, (copy_kernel<16, P>));             \
   MB_REGISTER_KERNEL("copy_edges_vpt1" SUFFIX, (copy_edges_kernel<1, P>));                  \
   MB_REGISTER_KERNEL("copy_edges_vpt2" SUFFIX, (copy_edges_kernel<2, P>));                  \
   MB_REGISTER_KERNEL("copy_edges_vpt4" SUFFIX, (copy_edges_kernel<4, P>));                  \
@@ -400,9 +399,9 @@ MB_REGISTER_KERNEL("fill_dwordx4", (fill_kernel<kPlain>));
 MB_REGISTER_KERNEL("fill_dwordx4_nt", (fill_kernel<kNontemporal>));
 MB_REGISTER_KERNEL("fill_dwordx4_stream", (fill_kernel<kStream>));
 MB_REGISTER_KERNEL("fill_tail", fill_tail_kernel);
-MB_REGISTER_KERNEL("read_sum_f32_vec", (read_sum_kernel<float, 4>));
-MB_REGISTER_KERNEL("read_sum_f16_vec", (read_sum_kernel<_Float16, 8>));
-MB_REGISTER_KERNEL("read_sum_bf16_vec", (read_sum_kernel<uint16_t, 8>));
+MB_REGISTER_KERNEL("read_sum_f32_vec", (read_sum_kernel<float>));
+MB_REGISTER_KERNEL("read_sum_f16_vec", (read_sum_kernel<_Float16>));
+MB_REGISTER_KERNEL("read_sum_bf16_vec", (read_sum_kernel<uint16_t>));
 #define MB_REGISTER_READ_PACKED(T, TNAME)                                            \
   MB_REGISTER_KERNEL("read_sum_" TNAME "_packed8", (read_sum_packed_kernel<T, 8>));     \
   MB_REGISTER_KERNEL("read_sum_" TNAME "_packed16", (read_sum_packed_kernel<T, 16>));   \
@@ -441,7 +440,7 @@ int launch_read(const void* src, float* sink, uint64_t elements, uint32_t block_
     case 64: read_sum_packed_kernel<T, 64><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
     case 128: read_sum_packed_kernel<T, 128><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
     case 256: read_sum_packed_kernel<T, 256><<<g, b, 0, stream>>>(s, sink, elements, chunks, serial); break;
-    default: read_sum_kernel<T, kVec><<<g, b, 0, stream>>>(s, sink, elements, block_elements, segments, serial);
+    default: read_sum_kernel<T><<<g, b, 0, stream>>>(s, sink, elements, block_elements, segments, serial);
   }
   return launch_status("read_sum_kernel");
 }

@@ -264,7 +264,8 @@ def run_gemm(args, metadata: dict, device) -> None:
                    **descriptor, **row_rates,
                    "config": {"block_m": config["tile_m"], "block_n": config["tile_n"], "block_k": config["tile_k"],
                               "threads": config["threads"]},
-                   "kernel": kernel, "tile_selection": "exact" if exact_tile else "automatic", "status": "ok", "correctness": correctness, "compiled": info,
+                   "kernel": kernel, "tile_selection": "exact" if exact_tile else "automatic", "status": "ok",
+                   "correctness": correctness, "compiled": info,
                    "roofline": roofline.describe(f"tensor_{dtype}", row_rates["peak_teraops_per_second"]),
                    **timing}
             rows.append(row)
