@@ -239,8 +239,9 @@ int mb_gemm_exact_tile(int format, const mb_gemm_config* config, const void* a, 
                        uint32_t group_m, void* stream);
 
 /* Registered name of the kernel mb_gemm launches for this call (of the
- * requested tile or a smaller one; "_checked" for rows too long for the fast
- * kernels' 32-bit offsets), for the instruction and resource audit of what actually runs; NULL
+ * requested tile or a smaller one; "_checked" where rows, a tile's rows of C or
+ * MXFP4 scale blocks exceed the fast kernels' 32-bit offsets, or MXFP4 scales are
+ * not on dwords), for the instruction and resource audit of what actually runs; NULL
  * with mb_last_error() set for an invalid call.
  * Replaces: the CompiledKernel the reference's launch returns for its audit
  * (bench_tensor.py:594-600, 988). */

@@ -54,7 +54,7 @@ def test_shapes_reach_every_kernel_of_any_shape(dtype):
 @pytest.mark.parametrize("dtype", FORMATS)
 def test_a_launch_never_exceeds_the_requested_tile(dtype):
     """Whatever the shape, the launched kernel's tile fits inside the requested one, and rows too long for
-    32-bit offsets go to the checked kernel."""
+    32-bit offsets, one of the checked kernel's cases, go to it."""
     for config in _configs(dtype):
         for m, n, k in [(1, 1, 256), (300, 5000, 512), (4096, 4096, 4096), (8192, 256, 1024)]:
             tile = _launched(dtype, config, m, n, k).split("_")[2]

@@ -16,7 +16,7 @@
 // among those with tiles no larger than the caller asked for:
 //   * gemm_dma_kernel (BF16, FP16, INT8, FP8, FP32 on 16x16 MFMAs),
 //     gemm_dma_f64_kernel and gemm_staged_kernel (MXFP4): 256x256 tiles
-//     (FP64 256x128) when the shape divides the tile. Four waves, one per SIMD,
+//     (FP64 256x128) when the tile divides the shape. Four waves, one per SIMD,
 //     each owning 128x128 outputs in AGPRs: 64 accumulators of 16x16 (the 16x16
 //     instructions sustain a higher clock under the power limit) or, for MXFP4,
 //     16 of 32x32. In the staged kernel operands flow global -> VGPR -> LDS ->
@@ -33,7 +33,8 @@
 //     64 tiles of 256x256 (39.3 us) but 256 of 128x128 (20.4 us).
 //   * gemm_kernel: 128x128 tiles staged through registers into a padded,
 //     double-buffered LDS tile, every load and store bounded with 64-bit
-//     addresses: rows too long for the other families' 32-bit offsets.
+//     addresses: rows, a tile's rows of C or MXFP4 scale blocks beyond the other
+//     families' 32-bit offsets, and MXFP4 scales off the dword grid.
 // All number workgroups XCD-first: the hardware deals consecutive ids
 // round-robin over the 8 XCDs, so ids are remapped to give each XCD a
 // contiguous share, walked in GROUP_M-row bands that keep A and B panels hot
@@ -955,7 +956,7 @@ const GemmKernel kRaggedKernels[] = {
     MB_RAGGED(MB_MATRIX_I8, MfmaI8x16, 7, "gemm_i8_256x256x128_ragged"),
 };
 
-// Any shape whose rows are too long for the ring kernels' 32-bit offsets.
+// Any shape: what the others' 32-bit offsets or dword-aligned scales exclude.
 #define MB_CHECKED(FMT, OP, NAME)                                                                             \
   GemmKernel {                                                                                                \
     FMT, 128, 128, 8, 1, GemmCost{}, NAME,                                                                    \

@@ -39,9 +39,16 @@ struct GemmKernel {
   GemmLauncher launch;
 };
 
-// Fitted to 317 launches on an MI355X (M, N from 256 to 8192, 2 to 64 K steps;
-// BF16, FP8 and MXFP4 together). Picking the cheapest estimate costs 0.7% on average against
-// always picking the fastest kernel; always taking the largest tile costs 126%.
+// BF16, FP16, FP8 and INT8, fitted to 317 launches on an MI355X (M, N from 256 to
+// 8192, 2 to 64 K steps) when the ring kernels were first written. On the kernels
+// as they are, over 4800 shapes (M, N from 32 to 11000, 1 to 370 steps), the
+// cheapest estimate runs the fastest kernel or one within 2% of it in 88 to 93% of
+// them and costs 0.7 (BF16) to 1.1% (FP8) on average; always 256x256 costs 143%.
+// One launch in 73 loses over 15%, typically 2.4 us, mostly on 64x64 tiles of which
+// a CU has two or three where one of 128x128 is faster; the worst are 54% (6.7 us)
+// and 98 us (15%). The ragged 256x256 kernel shares kCost256: where both can
+// run it takes 0.94 to 1.04 times the exact one's time. Tables:
+// profiles/gemm_dispatch.md.
 constexpr GemmCost kCost256{7.4f, 0.85f, 1.41f, false};
 constexpr GemmCost kCost256x128{4.5f, 0.44f, 0.855f, false};
 constexpr GemmCost kCost128{2.9f, 0.255f, 0.48f, false};
