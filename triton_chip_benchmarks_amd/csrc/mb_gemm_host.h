@@ -47,8 +47,7 @@ struct GemmKernel {
 // One launch in 73 loses over 15%, typically 2.4 us, mostly on 64x64 tiles of which
 // a CU has two or three where one of 128x128 is faster; the worst are 54% (6.7 us)
 // and 98 us (15%). The ragged 256x256 kernel shares kCost256: where both can
-// run it takes 0.94 to 1.04 times the exact one's time. Tables:
-// profiles/gemm_dispatch.md.
+// run it takes 0.94 to 1.04 times the exact one's time.
 constexpr GemmCost kCost256{7.4f, 0.85f, 1.41f, false};
 constexpr GemmCost kCost256x128{4.5f, 0.44f, 0.855f, false};
 constexpr GemmCost kCost128{2.9f, 0.255f, 0.48f, false};
